@@ -60,9 +60,67 @@ LUMX_HD f3 operator*(float s, f3 a) { return {s * a.x, s * a.y, s * a.z}; }
 LUMX_HD f3 operator/(f3 a, float s) { return {a.x / s, a.y / s, a.z / s}; }
 LUMX_HD f3 operator-(f3 a) { return {-a.x, -a.y, -a.z}; }
 LUMX_HD float dot3(f3 a, f3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+// Correctly rounded quotients without the compiler's range handling
+// (v_div_scale, v_div_fixup: 10 instructions a quotient).  With operands and
+// quotient far from the ends of the exponent range the residuals below are
+// exact, and Markstein's theorems (IBM J. Res. Dev. 34, 1990) give the IEEE
+// result: a Newton step with FMA takes a 1-ulp reciprocal to the correctly
+// rounded one, and a residual step takes a quotient within 1 ulp to the
+// correctly rounded one (the step before it brings a * inv there).  Checked
+// against IEEE division on gfx950 for every significand of d in rcp_rn, and
+// for 2^36 pairs in div_rn.  Three quotients by one divisor cost 18
+// instructions instead of 30.
+constexpr float kTiny = 0x1p-60f, kHuge = 0x1p60f;
+
+// 1 / d for kTiny <= |d| <= kHuge.
+LUMX_HD float rcp_rn(float d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float y = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, y, 1.0f), y, y);
+#else
+    return 1.0f / d;
+#endif
+}
+
+// a / d for kTiny <= |d| <= kHuge and a = 0 or kTiny <= |a| <= kHuge, with
+// inv = 1 / d correctly rounded.
+LUMX_HD float div_rn(float a, float d, float inv) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    float q = a * inv;
+    q = fmaf(fmaf(-d, q, a), inv, q);
+    return fmaf(fmaf(-d, q, a), inv, q);
+#else
+    (void)inv;
+    return a / d;
+#endif
+}
+
+// Square root of kTiny <= x <= kHuge: coupled Newton iteration for sqrt(x)
+// and 1 / (2 sqrt(x)) with a final residual step (Markstein 1990), equal to
+// the IEEE root for every significand and both exponent parities.
+LUMX_HD float sqrt_rn(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float y = __builtin_amdgcn_rsqf(x);
+    float g = x * y, h = 0.5f * y;
+    const float r = fmaf(-h, g, 0.5f);
+    g = fmaf(g, r, g);
+    h = fmaf(h, r, h);
+    return fmaf(fmaf(-g, g, x), h, g);
+#else
+    return sqrtf(x);
+#endif
+}
+
 LUMX_HD f3 normalize3(f3 v) {
     float len = sqrtf(dot3(v, v));
     return {v.x / len, v.y / len, v.z / len};
+}
+
+// normalize3 of a vector whose length and components lie in the range of
+// sqrt_rn and div_rn.
+LUMX_HD f3 normalize3_near1(f3 v) {
+    const float len = sqrt_rn(dot3(v, v)), inv = rcp_rn(len);
+    return {div_rn(v.x, len, inv), div_rn(v.y, len, inv), div_rn(v.z, len, inv)};
 }
 
 struct WorldView {
@@ -286,11 +344,16 @@ struct RayHit {
 struct MarchRay {
     f3 o, d, inv, corner;
 };
+LUMX_HD bool div_range(f3 v) {
+    return fminf(fminf(fabsf(v.x), fabsf(v.y)), fabsf(v.z)) >= kTiny &&
+           fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fabsf(v.z)) <= kHuge;
+}
 LUMX_HD MarchRay march_ray(f3 o, f3 d) {
     MarchRay m;
     m.o = o;
     m.d = d;
-    m.inv = {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
+    m.inv = {rcp_rn(d.x), rcp_rn(d.y), rcp_rn(d.z)};
+    if (!div_range(d)) m.inv = {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};  // axis-parallel rays, NaN
     m.corner = {d.x > 0.0f ? 16.0f : 0.0f, d.y > 0.0f ? 16.0f : 0.0f, d.z > 0.0f ? 16.0f : 0.0f};
     return m;
 }
@@ -344,8 +407,11 @@ LUMX_HD RayHit refine_hit(const WorldView& w, const MarchRay& m, float fraction)
     f3 bh = o + d * (fraction - 1.5f);
     int sx = d.x > 0.0f ? 1 : -1, sy = d.y > 0.0f ? 1 : -1, sz = d.z > 0.0f ? 1 : -1;
     f3 fl = {floorf(bh.x), floorf(bh.y), floorf(bh.z)};
-    f3 c1 = {(fl.x - bh.x) / d.x, (fl.y - bh.y) / d.y, (fl.z - bh.z) / d.z};
-    f3 c2 = {(fl.x - bh.x) / d.x + inv.x, (fl.y - bh.y) / d.y + inv.y, (fl.z - bh.z) / d.z + inv.z};
+    const f3 a = {fl.x - bh.x, fl.y - bh.y, fl.z - bh.z};
+    f3 c1 = {div_rn(a.x, d.x, inv.x), div_rn(a.y, d.y, inv.y), div_rn(a.z, d.z, inv.z)};
+    // a is 0, or bh itself within 1 of 0, or at least an ulp of |bh| >= 1.
+    if (!(div_range(d) && div_range(bh))) c1 = {a.x / d.x, a.y / d.y, a.z / d.z};
+    f3 c2 = {c1.x + inv.x, c1.y + inv.y, c1.z + inv.z};
     f3 tMax = {fmaxf(c1.x, c2.x), fmaxf(c1.y, c2.y), fmaxf(c1.z, c2.z)};
     // 1/|d| == |1/d| exactly (round-to-nearest is sign-symmetric).
     f3 tDelta = {fabsf(inv.x), fabsf(inv.y), fabsf(inv.z)};

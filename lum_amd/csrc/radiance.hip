@@ -18,7 +18,9 @@
 
 namespace lumx {
 
-__device__ __forceinline__ void hash33(uint32_t x, uint32_t y, uint32_t z, f3* out) {
+// hash33 mapped to [-1, 1]: (hash33 - 0.5) * 2 per component.  hash33's float
+// is (float)x * 2^-32, exact, so RN(x 2^-32 - 0.5) * 2 = RN(x 2^-31 - 1).
+__device__ __forceinline__ f3 hash33_signed(uint32_t x, uint32_t y, uint32_t z) {
     const uint32_t k = 1103515245u;
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
@@ -29,8 +31,7 @@ __device__ __forceinline__ void hash33(uint32_t x, uint32_t y, uint32_t z, f3* o
         y = ny;
         z = nz;
     }
-    const float inv = 2.3283064365386963e-10f;  // 1.0 / float(0xffffffffu) == 2^-32
-    *out = {(float)x * inv, (float)y * inv, (float)z * inv};
+    return {fmaf((float)x, 0x1p-31f, -1.0f), fmaf((float)y, 0x1p-31f, -1.0f), fmaf((float)z, 0x1p-31f, -1.0f)};
 }
 
 // total / R.  For R a power of two the quotient is total scaled by 2^-k,
@@ -92,17 +93,20 @@ __device__ __forceinline__ void ray_setup(const RadianceArgs& a, int key, int r,
     const int R = a.rays;
     const uint32_t t = (uint32_t)a.time_seed;
     const uint32_t gidx = (uint32_t)key * (uint32_t)R + (uint32_t)r;
-    f3 r0, r1;
-    hash33(gidx + t, t, t, &r0);
-    hash33(gidx + t + 1u, t, t, &r1);
+    const f3 j0 = hash33_signed(gidx + t, t, t);
+    const f3 j1 = hash33_signed(gidx + t + 1u, t, t);
     const float4 fb = gld(a.fib, (size_t)r);
-    f3 corner = f3{(float)px, (float)py, (float)pz} * 16.0f;
-    f3 center = corner + f3{8.0f, 8.0f, 8.0f};
-    const f3 half = {0.5f, 0.5f, 0.5f};
-    f3 dir = normalize3(f3{fb.x, fb.y, fb.z} + 0.1f * ((r0 - half) * 2.0f));
+    // Block centres are integers below 2^17, exact.
+    const f3 center = {(float)(px * 16 + 8), (float)(py * 16 + 8), (float)(pz * 16 + 8)};
+    // |fb| is 1 and each jitter component at most 0.1, so the length is
+    // within 0.82..1.18; a non-zero component is at least an ulp of the
+    // smallest jitter, 2^-60.
+    f3 dir = normalize3_near1(f3{fb.x, fb.y, fb.z} + 0.1f * j0);
     f3 pos = center + dir * 6.0f;
-    pos = pos + (r1 - half) * 2.0f;
-    if (r & 1) dir = -dir;
+    pos = pos + j1;
+    const uint32_t flip = (uint32_t)r << 31;  // odd lanes march the other way
+    dir = {__uint_as_float(__float_as_uint(dir.x) ^ flip), __uint_as_float(__float_as_uint(dir.y) ^ flip),
+           __uint_as_float(__float_as_uint(dir.z) ^ flip)};
     *pos_out = pos;
     *dir_out = dir;
 }
@@ -944,7 +948,6 @@ __global__ void __launch_bounds__(1024) radiance_tiled_kernel(RadianceArgs a) {
     occ.palette_slots = PB_LDS ? a.pb_words / 128 : wv.palette_slots;
     occ.block0_empty = wv.block0_empty;
     const int C = R < 64 ? R : 64;
-    const uint32_t t = (uint32_t)a.time_seed;
 
     while (true) {
         __syncthreads();  // staging done / previous batch fully consumed
@@ -972,18 +975,8 @@ __global__ void __launch_bounds__(1024) radiance_tiled_kernel(RadianceArgs a) {
                         (unsigned)pz < (unsigned)wv.wz;
             }
             if (valid) {
-                const uint32_t gidx = (uint32_t)wg * (uint32_t)R + (uint32_t)l;
-                f3 r0, r1;
-                hash33(gidx + t, t, t, &r0);
-                hash33(gidx + t + 1u, t, t, &r1);
-                const float4 fb = a.fib[l];
-                f3 corner = f3{(float)px, (float)py, (float)pz} * 16.0f;
-                f3 center = corner + f3{8.0f, 8.0f, 8.0f};
-                const f3 half = {0.5f, 0.5f, 0.5f};
-                f3 dir = normalize3(f3{fb.x, fb.y, fb.z} + 0.1f * ((r0 - half) * 2.0f));
-                f3 pos = center + dir * 6.0f;
-                pos = pos + (r1 - half) * 2.0f;
-                if (l & 1) dir = -dir;
+                f3 pos, dir;
+                ray_setup(a, wg, l, px, py, pz, &pos, &dir);
                 RayHit h = cast_ray_occ(occ, pos, dir, a.max_dist, a.max_steps);
                 if (h.hit) {
                     const float* m = s_mats + h.voxel * 6;
