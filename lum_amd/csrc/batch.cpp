@@ -316,6 +316,8 @@ int launcher_map(Launcher* L, lumx_world* const* worlds, int n, const int* n_mod
     for (int i = 0; i < m; ++i) n_launches = std::max(n_launches, ends[i].size());
     // Staging layout.
     std::vector<MapWorldDesc> desc(m);
+    std::vector<GridArgs> grids(m);
+    for (int i = 0; i < m; ++i) grids[i] = grid_args(worlds[i]);
     size_t off = round_up((size_t)m * sizeof(MapWorldDesc), 256);
     std::vector<size_t> launch_off(n_launches), launch_begin_off(n_launches);
     std::vector<int> launch_count(n_launches, 0);
@@ -341,6 +343,7 @@ int launcher_map(Launcher* L, lumx_world* const* worlds, int n, const int* n_mod
         d.empty_bits = w->empty_bits;
         d.palette = w->palette;
         d.pal_bits = w->pal_bits;
+        d.slot_mask = w->slot_mask;
         d.n_blocks = w->n_blocks;
         d.st = st;
         d.hi = std::max(hi, st);
@@ -424,6 +427,7 @@ int launcher_map(Launcher* L, lumx_world* const* worlds, int n, const int* n_mod
         HIP_TRY(launch_map_batch((const MapArgs*)(dv + launch_off[k]), (const int*)(dv + launch_begin_off[k]),
                                  launch_count[k], total_groups[k], s));
     HIP_TRY(launch_palette_bits_batch(d_dev, m, (int)slots, s));
+    HIP_TRY(launch_march_grid_batch(grids.data(), m, s));
     for (int i = 0; i < m; ++i) {
         worlds[i]->prev_counter = worlds[i]->counter;
         worlds[i]->ev_valid[1] = false;  // batched maps are not timed per world

@@ -10,6 +10,8 @@
 // the sequence (model, z, y, x) restricted to those first touches.  On the
 // device that is an ordered stream compaction over the concatenated boxes:
 //
+//   blockify_start_kernel    the current world is a copy of the origin world,
+//                            every claim idle;
 //   blockify_claim_kernel    every (model, block) element whose block has a
 //                            static origin id claims the block with atomicMin
 //                            of its model index;
@@ -19,12 +21,11 @@
 //   blockify_scan_kernel     one workgroup: tile offsets, the new counter, the
 //                            copy bound max(counter, previous counter);
 //   blockify_scatter_kernel  slot = static + offset + rank: the block's new id,
-//                            the slot's copy source, the claim released;
+//                            the slot's copy source;
 //   copy_bounded_kernel      exec_copies over the slots below the copy bound:
 //                            copy from the source block (0 = zero fill), zero
 //                            fill above the new counter.
-// The current world starts as a device copy of the origin world, so no world
-// crosses PCIe.
+// No world crosses PCIe.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -44,6 +45,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kTile = 2048;
+constexpr int kClaimIdle = 0x7fffffff;  // above every model index
 
 __global__ __launch_bounds__(64) void blockify_desc_kernel(BlockifyDesc d, int4* boxes, int* first) {
     const int i = threadIdx.x;
@@ -66,6 +68,23 @@ __device__ __forceinline__ void element(const BlockifyArgs& a, int t, int* m_out
     const int lx = l % ext.x, ly = (l / ext.x) % ext.y, lz = l / (ext.x * ext.y);
     *m_out = lo;
     *b_out = (unsigned)(bmin.x + lx) + (unsigned)a.wx * ((unsigned)(bmin.y + ly) + (unsigned)a.wy * (unsigned)(bmin.z + lz));
+}
+
+// start_blockify: the current world is the origin world, no block claimed.
+// Eight blocks a thread (every part of a world is 256-byte aligned).
+__global__ __launch_bounds__(kThreads) void blockify_start_kernel(BlockifyArgs a) {
+    const int j = (blockIdx.x * kThreads + threadIdx.x) * 8;
+    if (j + 8 <= a.n_blocks) {
+        *(uint4*)(a.blocks + j) = *(const uint4*)(a.origin + j);
+        const int4 idle = make_int4(kClaimIdle, kClaimIdle, kClaimIdle, kClaimIdle);
+        *(int4*)(a.claim + j) = idle;
+        *(int4*)(a.claim + j + 4) = idle;
+    } else {
+        for (int k = j; k < a.n_blocks; ++k) {
+            a.blocks[k] = a.origin[k];
+            a.claim[k] = kClaimIdle;
+        }
+    }
 }
 
 __global__ __launch_bounds__(kThreads) void blockify_claim_kernel(BlockifyArgs a) {
@@ -172,7 +191,6 @@ __global__ __launch_bounds__(kThreads) void blockify_scatter_kernel(BlockifyArgs
             a.copy_src[slot] = a.origin[b];
             a.blocks[b] = (int16_t)slot;
         }
-        a.claim[b] = a.claim_idle;
     }
 }
 
@@ -194,6 +212,8 @@ __global__ __launch_bounds__(256) void copy_bounded_kernel(uint8_t* palette, con
 size_t blockify_tiles(int n_elements) { return (size_t)(n_elements + kTile - 1) / kTile; }
 
 hipError_t launch_blockify(const BlockifyArgs& a, int copy_slots, hipStream_t stream) {
+    hipLaunchKernelGGL(blockify_start_kernel, dim3((a.n_blocks + 8 * kThreads - 1) / (8 * kThreads)), dim3(kThreads), 0,
+                       stream, a);
     if (a.n_elements > 0) {
         const int groups = (a.n_elements + kThreads - 1) / kThreads;
         hipLaunchKernelGGL(blockify_claim_kernel, dim3(groups), dim3(kThreads), 0, stream, a);

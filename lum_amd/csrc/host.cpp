@@ -219,6 +219,22 @@ WorldView lumx::view_of(const lumx_world* w) {
     return v;
 }
 
+GridArgs lumx::grid_args(const lumx_world* w) {
+    GridArgs g;
+    g.empty_bits = w->empty_bits;
+    g.blocks = w->blocks;
+    g.slot_mask = w->slot_mask;
+    g.slots = w->desc.palette_slots;
+    g.grid = w->grid;
+    g.escape = w->escape;
+    g.wx = w->desc.size[0];
+    g.wy = w->desc.size[1];
+    g.wz = w->desc.size[2];
+    g.n_blocks = w->n_blocks;
+    g.tiles = w->grid ? march_grid_tiles(g.wx, g.wy, g.wz) : 0;
+    return g;
+}
+
 // ---------------------------------------------------------------------------
 // C ABI
 // ---------------------------------------------------------------------------
@@ -291,7 +307,7 @@ void* lumx_context_stream(lumx_context_t c) { return c ? (void*)c->stream : null
 // only changes fields, so a server copies that range out once).
 struct WorldLayout {
     size_t blocks, copy_src, mats, palette, field0, field1, empty_bits, pal_bits, batch_counter, sel_bits,
-        sel_tiles, sel_claim, upd_claim, upd_tiles, origin, blockify_state, total;
+        sel_tiles, block_claim, upd_claim, upd_tiles, origin, blockify_state, total;
 };
 
 static WorldLayout world_layout(const lumx_world* w) {
@@ -315,7 +331,7 @@ static WorldLayout world_layout(const lumx_world* w) {
     L.batch_counter = take(2 * sizeof(unsigned int));
     L.sel_bits = take(lumx::select_bits_bytes(w->n_blocks));
     L.sel_tiles = take(lumx::select_tiles(w->n_blocks) * sizeof(int));
-    L.sel_claim = take(nb * sizeof(int));
+    L.block_claim = take(nb * sizeof(int));
     L.upd_claim = take(nb * sizeof(int));
     L.upd_tiles = take((lumx::select_tiles(w->n_blocks) + 1) * sizeof(int));
     L.origin = take(nb * sizeof(int16_t));
@@ -337,7 +353,20 @@ static void world_carve(lumx_world* w, char* base) {
     w->batch_counter = (unsigned int*)(base + L.batch_counter);
     w->sel_bits = (unsigned long long*)(base + L.sel_bits);
     w->sel_tiles = (int*)(base + L.sel_tiles);
-    w->sel_claim = (int*)(base + L.sel_claim);
+    w->block_claim = (int*)(base + L.block_claim);
+    // Escape masks, then the padded grid, in the claim words (the march forms
+    // grid indices in floats, exact below 2^24).
+    const long long nb = w->n_blocks, padded = (long long)(w->desc.size[0] + 2) * (w->desc.size[1] + 2) *
+                                               (w->desc.size[2] + 2);
+    const bool fits = nb + padded <= 4 * nb && padded <= (1 << 24);
+    w->escape = fits ? (uint8_t*)w->block_claim : nullptr;
+    w->grid = fits ? w->escape + nb : nullptr;
+    // Octants of the slots, where they fit as well (worlds in which the march's
+    // margin of 1/256 voxel covers the rounding of positions).
+    const int* ws = w->desc.size;
+    w->slot_mask = fits && nb + padded + w->desc.palette_slots <= 4 * nb && std::max(ws[0], std::max(ws[1], ws[2])) <= 512
+                       ? w->grid + padded
+                       : nullptr;
     w->upd_claim = (int*)(base + L.upd_claim);
     w->upd_tiles = (int*)(base + L.upd_tiles);
     w->origin_dev = (int16_t*)(base + L.origin);
@@ -376,8 +405,7 @@ static lumx::AttachArgs attach_args(lumx_world* w, int used) {
     a.n_blocks = w->n_blocks;
     a.empty_bits = w->empty_bits;
     a.pal_bits = w->pal_bits;
-    a.sel_claim = w->sel_claim;
-    a.claim_idle = lumx::select_claim_idle();
+    a.slot_mask = w->slot_mask;
     a.upd_claim = w->upd_claim;
     a.batch_counter = w->batch_counter;
     a.blockify_state = w->blockify_state;
@@ -391,7 +419,8 @@ static lumx::AttachArgs attach_args(lumx_world* w, int used) {
 // counters zero (the map counter `counter`), occupancy bits rebuilt from the
 // blocks and the palette (one kernel on s).
 static hipError_t world_init_rest(lumx_world* w, int used, hipStream_t s) {
-    return lumx::launch_world_attach(attach_args(w, used), s);
+    hipError_t e = lumx::launch_world_attach(attach_args(w, used), s);
+    return e == hipSuccess ? lumx::launch_march_grid(lumx::grid_args(w), s) : e;
 }
 
 // A world's own device block, every part zeroed (claims and counters idle).
@@ -434,7 +463,8 @@ static void world_free_device(lumx_world* w) {
     w->batch_counter = nullptr;
     w->sel_bits = nullptr;
     w->sel_tiles = nullptr;
-    w->sel_claim = nullptr;
+    w->block_claim = nullptr;
+    w->grid = w->escape = w->slot_mask = nullptr;
     w->upd_claim = nullptr;
     w->origin_dev = nullptr;
     w->blockify_state = nullptr;
@@ -523,6 +553,9 @@ int lumx::world_attach_init_many(lumx_world* const* ws, int n, hipStream_t s) {
     std::vector<lumx::AttachArgs> a((size_t)n);
     for (int i = 0; i < n; ++i) a[i] = attach_args(ws[i], ws[i]->snap_used);
     HIP_TRY(lumx::launch_world_attach_batch(a.data(), n, s));
+    std::vector<lumx::GridArgs> g((size_t)n);
+    for (int i = 0; i < n; ++i) g[i] = lumx::grid_args(ws[i]);
+    HIP_TRY(lumx::launch_march_grid_batch(g.data(), n, s));
     return LUMX_OK;
 }
 
@@ -688,7 +721,8 @@ int lumx_world_set_palette(lumx_world_t w, int first, int count, const uint8_t* 
         if (w->static_palette[i]) { e0 = false; break; }
     w->block0_empty = e0;
     HIP_TRY(hipMemcpy(w->palette + (size_t)first * 4096, tmp.data(), tmp.size(), hipMemcpyHostToDevice));
-    HIP_TRY(launch_palette_bits(w->palette, first, count, w->pal_bits, nullptr));
+    HIP_TRY(launch_palette_bits(w->palette, first, count, w->pal_bits, w->slot_mask, 0, nullptr));
+    HIP_TRY(launch_march_grid(grid_args(w), nullptr));
     HIP_TRY(hipDeviceSynchronize());
     return LUMX_OK;
 }
@@ -849,7 +883,8 @@ static int sync_host_state(lumx_world* w) {
 static int commit_palette_bits(lumx_world* w, hipStream_t s) {
     const int st = w->desc.static_blocks;
     const int hi = std::max(w->counter, w->prev_counter);
-    if (hi > st) HIP_TRY(launch_palette_bits(w->palette, st, hi - st, w->pal_bits, s));
+    if (hi > st) HIP_TRY(launch_palette_bits(w->palette, st, hi - st, w->pal_bits, w->slot_mask, 0, s));
+    HIP_TRY(launch_march_grid(grid_args(w), s));
     w->prev_counter = w->counter;
     return LUMX_OK;
 }
@@ -1272,15 +1307,13 @@ static int map_device(lumx_world_t w, int n, const lumx_model_t* models, const l
         // A recorded upload runs only when the graph does: eager maps keep uploading.
         if (!capturing) w->origin_dirty = false;
     }
-    // start_blockify: the current world is the origin world.
-    HIP_TRY(hipMemcpyAsync(w->blocks, w->origin_dev, (size_t)w->n_blocks * 2, hipMemcpyDeviceToDevice, s));
     BlockifyArgs a{};
     a.origin = w->origin_dev;
     a.blocks = w->blocks;
     a.copy_src = w->copy_src_dev;
     a.palette = w->palette;
-    a.claim = w->sel_claim;
-    a.claim_idle = select_claim_idle();
+    a.claim = w->block_claim;
+    a.n_blocks = w->n_blocks;
     a.wx = w->desc.size[0];
     a.wy = w->desc.size[1];
     a.wz = w->desc.size[2];
@@ -1302,7 +1335,10 @@ static int map_device(lumx_world_t w, int n, const lumx_model_t* models, const l
     HIP_TRY(launch_block_bits(w->blocks, w->n_blocks, w->empty_bits, s));
     int rc = launch_models(w, n, models, pl, s);
     if (rc) return rc;
-    if (bound > st) HIP_TRY(launch_palette_bits(w->palette, st, bound - st, w->pal_bits, s));
+    // The claims took the place of every slot's mask.
+    const int from = w->slot_mask ? 0 : st, fill = w->slot_mask ? slots : 0;
+    HIP_TRY(launch_palette_bits(w->palette, from, bound - from, w->pal_bits, w->slot_mask, fill, s));
+    HIP_TRY(launch_march_grid(grid_args(w), s));
     w->host_stale = true;
     w->dev_counter_bound = (int)std::min<long long>(slots, st + total);
     if (capturing) return LUMX_OK;
@@ -1474,6 +1510,11 @@ int lumx::radiance_args(lumx_world* w, const int32_t* req, int n_req, const lumx
     a.pb_words = w->desc.palette_slots * 128;
     a.batch_counter = w->batch_counter;
     a.staged = (req != nullptr || p->size != 1) ? 1 : 0;
+    // The grid march takes slot 0 as air and rays no longer than its reach.
+    if (w->block0_empty && p->max_dist <= kGridMaxDist) {
+        a.grid = w->grid;
+        a.escape = w->escape;
+    }
     a.div_x = make_divisor((uint32_t)w->desc.size[0]);
     a.div_xy = make_divisor((uint32_t)w->desc.size[0] * (uint32_t)w->desc.size[1]);
     return LUMX_OK;

@@ -103,8 +103,13 @@ struct lumx_world {
     unsigned int* batch_counter = nullptr;  // device: tiled kernel work counter (2 words)
     unsigned long long* sel_bits = nullptr; // device probe selection: flags, one word per 64 probes
     int* sel_tiles = nullptr;               // device probe selection: per-tile counts / offsets
-    int* sel_claim = nullptr;               // per block claim word shared by probe selection and
-                                            // device blockify (idle between calls)
+    // Per block one word that the device blockify uses for its claims while it
+    // runs, and that holds the march grid and escape masks between maps
+    // (nullptr when the padded grid does not fit: worlds a few blocks wide).
+    int* block_claim = nullptr;
+    uint8_t* grid = nullptr;
+    uint8_t* escape = nullptr;
+    uint8_t* slot_mask = nullptr;
     int* upd_claim = nullptr;               // per probe: last request of a subset update that
                                             // named it (-1 between updates)
     int* upd_tiles = nullptr;               // compacted subset update: per tile of 2048 probes
@@ -198,6 +203,8 @@ void compact_args(const lumx_world* w, RadianceArgs* a);
 void glossy_args(lumx_world* w, const uint8_t* matnorm, const float* depth, int width, int height,
                  const lumx_camera* cam, float max_dist, int max_steps, float* out, int32_t* keys, GlossyArgs* a);
 WorldView view_of(const lumx_world* w);
+// The march grid of w's blocks, built from its empty-block bits.
+GridArgs grid_args(const lumx_world* w);
 bool stream_capturing(hipStream_t s);
 
 // Batched launches over any set of distinct worlds (batch.cpp).

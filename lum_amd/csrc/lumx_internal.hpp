@@ -50,7 +50,51 @@ struct RadianceArgs {
     int list_stride;             // texel bytes
     int* tiles;                  // per tile of 2048 texels: count, then offset; [n_tiles] = entries
     int n_tiles;
+    // March grid of the world (nullptr: not available, or the update's rays
+    // may be longer than kGridMaxDist).
+    const uint8_t* grid;
+    const uint8_t* escape;
 };
+
+// March grid: what the radiance march asks of the blocks, in one byte each.
+//   grid    (wx + 2)(wy + 2)(wz + 2) bytes, the world with one block of
+//           padding on every side: 0 where the block is in the world and
+//           empty, 0xff outside; else the octants (8^3 voxels) of the block
+//           that may hold a voxel, at least one of them;
+//   escape  one byte per block: bit (x < 0) + 2 (y < 0) + 4 (z < 0) is set
+//           when the 9 x 9 x 9 blocks from this one towards that octant are
+//           empty (or outside the world).  A ray of at most kGridMaxDist
+//           voxels that starts within 7 voxels of the block's centre and
+//           moves into that octant hits nothing: its samples reach 128.5 + 7
+//           voxels from the centre, so blocks at most 8 away, and rounding
+//           keeps every coordinate monotone along the ray.
+constexpr float kGridMaxDist = 128.0f;
+struct GridArgs {
+    const uint32_t* empty_bits;
+    const int16_t* blocks;
+    const uint8_t* slot_mask;  // per slot (nullptr: unknown): which of its 8^3 octants hold a voxel
+    uint8_t* grid;
+    uint8_t* escape;
+    int wx, wy, wz, n_blocks, slots;
+    int tiles;              // march_grid_tiles(wx, wy, wz)
+};
+#if defined(__HIPCC__)
+// Octants of a slot with a voxel, from its occupancy words (128 threads).
+__device__ __forceinline__ void slot_octants(uint32_t word, int slot, uint8_t* slot_mask) {
+    __shared__ unsigned upper;
+    const unsigned long long y0 = 0x0f0f0f0f0f0f0f0full;  // words of rows y < 8
+    const unsigned long long lo = __ballot((word & 0x00ff00ffu) != 0), hi = __ballot((word & 0xff00ff00u) != 0);
+    const unsigned m = ((lo & y0) != 0) | ((hi & y0) != 0) << 1 | ((lo & ~y0) != 0) << 2 | ((hi & ~y0) != 0) << 3;
+    if (threadIdx.x == 64) upper = m << 4;
+    __syncthreads();
+    if (threadIdx.x == 0) slot_mask[slot] = (uint8_t)(m | upper);
+}
+#endif
+int march_grid_tiles(int wx, int wy, int wz);
+hipError_t launch_march_grid(const GridArgs& g, hipStream_t stream);
+// Grids of n worlds, up to kGridBatch worlds a launch (descriptors by value).
+constexpr int kGridBatch = 32;
+hipError_t launch_march_grid_batch(const GridArgs* g, int n, hipStream_t stream);
 
 // Launch shape of the tiled radiance kernel (chosen by the autotuner).
 struct RadianceTune {
@@ -154,11 +198,11 @@ struct ShiftArgs {
 // Device blockify (blockify.hip).
 struct BlockifyArgs {
     const int16_t* origin;      // origin world (device)
-    int16_t* blocks;            // current world, a copy of origin on entry
+    int16_t* blocks;            // current world
     int32_t* copy_src;          // per slot: static source block
     uint8_t* palette;
-    int* claim;                 // per block: first model covering it, idle value otherwise
-    int claim_idle;
+    int* claim;                 // per block: first model covering it (this map's scratch)
+    int n_blocks;
     int wx, wy, wz;
     int static_count, palette_slots;
     int n_models, n_elements, n_tiles;
@@ -200,8 +244,7 @@ struct AttachArgs {
     int n_blocks;
     uint32_t* empty_bits;       // per block: 1 = id 0
     uint32_t* pal_bits;         // per slot: 128 words of voxel occupancy
-    int* sel_claim;
-    int claim_idle;
+    uint8_t* slot_mask;         // per slot: octants with a voxel (nullptr: the world has none)
     int* upd_claim;
     unsigned int* batch_counter;
     int* blockify_state;
@@ -214,7 +257,6 @@ hipError_t launch_world_attach_batch(const AttachArgs* a, int n, hipStream_t str
 
 size_t select_tiles(int n_probes);
 size_t select_bits_bytes(int n_probes);
-int select_claim_idle();
 hipError_t launch_select(const SelectArgs& a, hipStream_t stream);
 hipError_t launch_shift(const ShiftArgs& a, int texel_bytes, hipStream_t stream);
 
@@ -250,7 +292,7 @@ hipError_t launch_radiance_tiled(RadianceArgs a, int store, bool traced, const R
 hipError_t launch_radiance_refill(const RadianceArgs& a, int store, int P, hipStream_t stream);
 size_t radiance_tiled_lds_bytes(const RadianceArgs& a, const RadianceTune& t);
 hipError_t launch_block_bits(const int16_t* blocks, int n_blocks, uint32_t* bits, hipStream_t stream);
-hipError_t launch_palette_bits(const uint8_t* palette, int first_slot, int n_slots, uint32_t* bits,
+hipError_t launch_palette_bits(const uint8_t* palette, int first_slot, int n_slots, uint32_t* bits, uint8_t* slot_mask, int fill_end,
                                hipStream_t stream);
 hipError_t launch_map_group(const MapGroup& g, hipStream_t stream);
 
@@ -268,6 +310,7 @@ struct MapWorldDesc {
     uint32_t* empty_bits;
     uint8_t* palette;
     uint32_t* pal_bits;
+    uint8_t* slot_mask;       // nullptr: the world has none
     long long stage_origin;   // byte offset of the staged origin world, -1: the device copy is current
     unsigned long long stage_copy;    // byte offset of the staged copy list (slots st .. hi - 1)
     unsigned long long stage_slots;   // byte offset of the staged slot blocks (slots st .. counter - 1)

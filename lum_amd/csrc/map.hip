@@ -206,6 +206,7 @@ __global__ void __launch_bounds__(128) palette_bits_batch_kernel(const MapWorldD
 #pragma unroll
     for (int k = 0; k < 32; ++k) v |= (((words[k >> 2] >> ((k & 3) * 8)) & 0xffu) != 0 ? 1u : 0u) << k;
     w.pal_bits[((size_t)slot << 7) + threadIdx.x] = v;
+    if (w.slot_mask) slot_octants(v, slot, w.slot_mask);
 }
 
 // One workgroup of 256 threads per slot, 16 B per thread.

@@ -154,16 +154,19 @@ template <> struct Texel<STORE_F32> {
     typedef float4 type;
     LUMX_HD static f3 load(const void* base, unsigned i) {
         // 32-bit byte offsets: a field holds at most 2^28 texels of 16 B.
-        float4 v = gld((const float4*)((const char*)base + (i << 4)), 0);
-        return {v.x, v.y, v.z};
+        return unpack(gld((const float4*)((const char*)base + (i << 4)), 0));
     }
+    LUMX_HD static f3 unpack(float4 v) { return {v.x, v.y, v.z}; }
     LUMX_HD static void store(void* base, unsigned i, f3 v) {
         gst((float4*)((char*)base + (i << 4)), 0, make_float4(v.x, v.y, v.z, 1.0f));
     }
 };
 template <> struct Texel<STORE_F16> {
+    typedef uint2 type;
     LUMX_HD static f3 load(const void* base, unsigned i) {
-        uint2 raw = gld((const uint2*)((const char*)base + (i << 3)), 0);
+        return unpack(gld((const uint2*)((const char*)base + (i << 3)), 0));
+    }
+    LUMX_HD static f3 unpack(uint2 raw) {
         _Float16 h[4];
         __builtin_memcpy(h, &raw, 8);
         return {(float)h[0], (float)h[1], (float)h[2]};
@@ -176,8 +179,11 @@ template <> struct Texel<STORE_F16> {
     }
 };
 template <> struct Texel<STORE_BF16> {
+    typedef uint2 type;
     LUMX_HD static f3 load(const void* base, unsigned i) {
-        uint2 raw = gld((const uint2*)((const char*)base + (i << 3)), 0);
+        return unpack(gld((const uint2*)((const char*)base + (i << 3)), 0));
+    }
+    LUMX_HD static f3 unpack(uint2 raw) {
         return {bf16_to_f32((uint16_t)(raw.x & 0xffffu)), bf16_to_f32((uint16_t)(raw.x >> 16)),
                 bf16_to_f32((uint16_t)(raw.y & 0xffffu))};
     }
@@ -235,12 +241,16 @@ LUMX_HD int block_id(const WorldView& w, int bx, int by, int bz) {
     return gld((const int16_t*)((const char*)w.blocks + (lin << 1)), 0);
 }
 
+// Offset of voxel (ix, iy, iz) mod 16 within its palette slot.
+LUMX_HD uint32_t voxel_offset(int ix, int iy, int iz) {
+    return (uint32_t)((ix & 15) | ((iy & 15) << 4) | ((iz & 15) << 8));
+}
+
 // voxel_in_palette: voxel (ix, iy, iz) mod 16 of block b.
 LUMX_HD int voxel_in_block(const WorldView& w, int b, int ix, int iy, int iz) {
     if (b == 0 && w.block0_empty) return 0;
     if ((unsigned)b >= (unsigned)w.palette_slots) return 0;
-    uint32_t off = ((uint32_t)b << 12) | (uint32_t)((ix & 15) | ((iy & 15) << 4) | ((iz & 15) << 8));
-    return gld(w.palette, off);
+    return gld(w.palette, ((uint32_t)b << 12) | voxel_offset(ix, iy, iz));
 }
 
 // GetBlock + palette fetch for an integer voxel position.
@@ -290,17 +300,22 @@ LUMX_HD int wrap_next(int x, int n) {
     return (int)umin_(u, u - (unsigned)n);
 }
 
-// Trilinear LINEAR filter with REPEAT wrap at texel-space coordinate bp
-// (texel i's centre at bp = i, i.e. normalized coordinate (bp + 0.5) / size).
+LUMX_HD f3 trilinear(f3 t000, f3 t100, f3 t010, f3 t110, f3 t001, f3 t101, f3 t011, f3 t111, f3 t) {
+    const float ux = 1.0f - t.x, uy = 1.0f - t.y, uz = 1.0f - t.z;
+    const f3 c00 = t000 * ux + t100 * t.x;
+    const f3 c10 = t010 * ux + t110 * t.x;
+    const f3 c01 = t001 * ux + t101 * t.x;
+    const f3 c11 = t011 * ux + t111 * t.x;
+    const f3 c0 = c00 * uy + c10 * t.y;
+    const f3 c1 = c01 * uy + c11 * t.y;
+    return c0 * uz + c1 * t.z;
+}
+
+// The eight taps of the cell at (x0, y0, z0), weighted by t.
 template <int STORE>
-LUMX_HD f3 sample_texel(const void* field, int wx, int wy, int wz, f3 bp) {
-    float fx0 = floorf(bp.x), fy0 = floorf(bp.y), fz0 = floorf(bp.z);
-    float tx = bp.x - fx0, ty = bp.y - fy0, tz = bp.z - fz0;
-    int ix = (int)fx0, iy = (int)fy0, iz = (int)fz0;
+LUMX_HD f3 sample_taps(const void* field, int wx, int wy, int wz, int x0, int y0, int z0, f3 t) {
     // REPEAT: the second tap of each axis is the first one's successor mod n.
-    int x0 = wrap_i(ix, wx), x1 = wrap_next(x0, wx);
-    int y0 = wrap_i(iy, wy), y1 = wrap_next(y0, wy);
-    int z0 = wrap_i(iz, wz), z1 = wrap_next(z0, wz);
+    const int x1 = wrap_next(x0, wx), y1 = wrap_next(y0, wy), z1 = wrap_next(z0, wz);
     // Operands below 2^24 (axes <= 4096, wy * wz <= 2^24): 24-bit multiplies.
     const unsigned r00 = mul24((unsigned)wx, (unsigned)y0 + mul24((unsigned)wy, (unsigned)z0));
     const unsigned r10 = mul24((unsigned)wx, (unsigned)y1 + mul24((unsigned)wy, (unsigned)z0));
@@ -314,14 +329,17 @@ LUMX_HD f3 sample_texel(const void* field, int wx, int wy, int wz, f3 bp) {
     f3 t101 = Texel<STORE>::load(field, r01 + (unsigned)x1);
     f3 t011 = Texel<STORE>::load(field, r11 + (unsigned)x0);
     f3 t111 = Texel<STORE>::load(field, r11 + (unsigned)x1);
-    float ux = 1.0f - tx, uy = 1.0f - ty, uz = 1.0f - tz;
-    f3 c00 = t000 * ux + t100 * tx;
-    f3 c10 = t010 * ux + t110 * tx;
-    f3 c01 = t001 * ux + t101 * tx;
-    f3 c11 = t011 * ux + t111 * tx;
-    f3 c0 = c00 * uy + c10 * ty;
-    f3 c1 = c01 * uy + c11 * ty;
-    return c0 * uz + c1 * tz;
+    return trilinear(t000, t100, t010, t110, t001, t101, t011, t111, t);
+}
+
+// Trilinear LINEAR filter with REPEAT wrap at texel-space coordinate bp
+// (texel i's centre at bp = i, i.e. normalized coordinate (bp + 0.5) / size).
+template <int STORE>
+LUMX_HD f3 sample_texel(const void* field, int wx, int wy, int wz, f3 bp) {
+    float fx0 = floorf(bp.x), fy0 = floorf(bp.y), fz0 = floorf(bp.z);
+    float tx = bp.x - fx0, ty = bp.y - fy0, tz = bp.z - fz0;
+    int ix = (int)fx0, iy = (int)fy0, iz = (int)fz0;
+    return sample_taps<STORE>(field, wx, wy, wz, wrap_i(ix, wx), wrap_i(iy, wy), wrap_i(iz, wz), f3{tx, ty, tz});
 }
 
 // sample_radiance: trilinear at texel coordinate (x + n*16)/16, REPEAT wrap.

@@ -36,7 +36,6 @@ namespace {
 
 constexpr int kSelThreads = 256;
 constexpr int kSelTile = 2048;  // probes per tile: 8 per thread, 32 ballot words
-constexpr int kClaimIdle = 0x7f7f7f7f;
 
 __device__ __forceinline__ int neighbour_sum(const int16_t* blocks, int wx, int wy, int wz, int x, int y, int z) {
     int s = 0;
@@ -188,7 +187,6 @@ __global__ __launch_bounds__(256) void shift_kernel(ShiftArgs a) {
 
 size_t select_tiles(int n_probes) { return (size_t)(n_probes + kSelTile - 1) / kSelTile; }
 size_t select_bits_bytes(int n_probes) { return select_tiles(n_probes) * (kSelTile / 8); }
-int select_claim_idle() { return kClaimIdle; }
 
 hipError_t launch_select(const SelectArgs& a, hipStream_t stream) {
     if (a.n_tiles > 0)

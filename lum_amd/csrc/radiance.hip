@@ -88,13 +88,12 @@ __device__ __forceinline__ bool probe_coords(const RadianceArgs& a, int wg, int*
 
 // Ray r of the probe of request index `key` at block (px, py, pz)
 // (radiance.comp:370-381): origin and direction.
-__device__ __forceinline__ void ray_setup(const RadianceArgs& a, int key, int r, int px, int py, int pz,
+__device__ __forceinline__ void ray_setup(const RadianceArgs& a, int time_seed, int key, int r, int px, int py, int pz,
                                           f3* pos_out, f3* dir_out) {
-    const int R = a.rays;
-    const uint32_t t = (uint32_t)a.time_seed;
-    const uint32_t gidx = (uint32_t)key * (uint32_t)R + (uint32_t)r;
-    const f3 j0 = hash33_signed(gidx + t, t, t);
-    const f3 j1 = hash33_signed(gidx + t + 1u, t, t);
+    const uint32_t t = (uint32_t)time_seed;
+    const uint32_t seed = (uint32_t)key * (uint32_t)a.rays + t;
+    const f3 j0 = hash33_signed(seed + (uint32_t)r, t, t);
+    const f3 j1 = hash33_signed(seed + (uint32_t)r + 1u, t, t);
     const float4 fb = gld(a.fib, (size_t)r);
     // Block centres are integers below 2^17, exact.
     const f3 center = {(float)(px * 16 + 8), (float)(py * 16 + 8), (float)(pz * 16 + 8)};
@@ -111,6 +110,18 @@ __device__ __forceinline__ void ray_setup(const RadianceArgs& a, int key, int r,
     *dir_out = dir;
 }
 
+// Light of a ray that leaves the world (radiance.comp:333-344).
+__device__ __forceinline__ f3 sky_light(f3 dir) {
+    f3 light = {0.0f, 0.0f, 0.0f};
+    const float gl = -dot3(dir, radiance_light_dir());
+    if (gl > 0.95f) {
+        f3 sun = f3{0.9f, 0.9f, 0.6f} * 3.0f;
+        light = light + gl * sun;
+    }
+    f3 sky = f3{0.53f, 0.81f, 0.92f} * 0.1f;
+    return light + sky;
+}
+
 // trace_ray's shading of a cast ray from pos along dir (radiance.comp:316-347).
 template <int STORE>
 __device__ __forceinline__ f3 shade_ray(const RadianceArgs& a, const RayHit& h, f3 pos, f3 dir) {
@@ -121,13 +132,7 @@ __device__ __forceinline__ f3 shade_ray(const RadianceArgs& a, const RayHit& h, 
         f3 prop = sample_radiance<STORE>(a.field_in, w.wx, w.wy, w.wz, pos + h.fraction * dir, h.normal);
         light = light + (prop * m.color + m.color * m.emit);
     } else {
-        float gl = -dot3(dir, radiance_light_dir());
-        if (gl > 0.95f) {
-            f3 sun = f3{0.9f, 0.9f, 0.6f} * 3.0f;
-            light = light + gl * sun;
-        }
-        f3 sky = f3{0.53f, 0.81f, 0.92f} * 0.1f;
-        light = light + sky;
+        light = sky_light(dir);
     }
     return light;
 }
@@ -136,11 +141,11 @@ __device__ __forceinline__ f3 shade_ray(const RadianceArgs& a, const RayHit& h, 
 // (px, py, pz).  Traced launches (never compacted: key is the probe's index
 // in the launch) record the ray at key * R + r.
 template <int STORE, bool TRACED, bool OCC>
-__device__ __forceinline__ f3 probe_ray_light(const RadianceArgs& a, int key, int r, int px, int py, int pz) {
+__device__ __forceinline__ f3 probe_ray_light(const RadianceArgs& a, int time_seed, int key, int r, int px, int py, int pz) {
     const WorldView& w = a.world;
     const int R = a.rays;
     f3 pos, dir;
-    ray_setup(a, key, r, px, py, pz, &pos, &dir);
+    ray_setup(a, time_seed, key, r, px, py, pz, &pos, &dir);
 
     RayHit h;
     if (OCC) {
@@ -233,7 +238,7 @@ __device__ __forceinline__ void store_probe(const RadianceArgs& a, int wg, int p
 //   or o = 0, 2, 1, 3 (Kw = 4): stage C/2 pairs rays p and p + C/2 (o = 0, 2
 //   for Kw = 4), stage C/4 pairs their sums.
 template <int STORE, bool TRACED, bool OCC, int K>
-__device__ __forceinline__ void radiance_lane_body(const RadianceArgs& a, const int tid, f3* chunk_sum) {
+__device__ __forceinline__ void radiance_lane_body(const RadianceArgs& a, const int time_seed, const int tid, f3* chunk_sum) {
     const int R = a.rays;
     constexpr int LOG2K = K == 1 ? 0 : (K == 2 ? 1 : 2);
     const int L = R >> LOG2K;  // K > 1: R is a power of two
@@ -247,7 +252,7 @@ __device__ __forceinline__ void radiance_lane_body(const RadianceArgs& a, const 
     const int C = R < 64 ? R : 64;
     f3 total;
     if (K == 1) {
-        f3 light = valid ? probe_ray_light<STORE, TRACED, OCC>(a, key, m, px, py, pz) : zero;
+        f3 light = valid ? probe_ray_light<STORE, TRACED, OCC>(a, time_seed, key, m, px, py, pz) : zero;
         total = butterfly(light, C);
         if (R > 64) {
             const int wave = threadIdx.x >> 6;
@@ -275,7 +280,7 @@ __device__ __forceinline__ void radiance_lane_body(const RadianceArgs& a, const 
             const int jc = j / Kw, jj = j - jc * Kw;
             const int o = Kw == 4 ? (((jj & 1) << 1) | (jj >> 1)) : jj;
             const int r = (g * Kc + jc) * C + p + o * Lc;
-            const f3 v = valid ? probe_ray_light<STORE, TRACED, OCC>(a, key, r, px, py, pz) : zero;
+            const f3 v = valid ? probe_ray_light<STORE, TRACED, OCC>(a, time_seed, key, r, px, py, pz) : zero;
             if (Kw == 1) {
                 cur = v;
             } else if (Kw == 2) {
@@ -318,10 +323,418 @@ __device__ __forceinline__ void radiance_lane_body(const RadianceArgs& a, const 
     if (valid && m == 0) store_probe<STORE>(a, wg, px, py, pz, total);
 }
 
+// Chunk waves: the default launch.  A wave traces 64 rays, one per lane, as in
+// radiance_lane_body and to the same bits, but in four parts:
+//   - what its rays share (the probe, its block, the field's cell, the fixed
+//     part of the hash) is loaded and computed on the scalar unit;
+//   - a ray that ends in its own block without a step (half the rays of a
+//     heightmap world) is shaded from the block's cell, without the march;
+//   - a ray whose octant of blocks is empty (most of the others) is sky;
+//   - what is left marches the world's grid of bytes (cast_ray_grid).
+// The march is bound by vector issue and by the latency of its gathers, so
+// waves in flight count: 80 scalar registers and 64 vector registers keep
+// eight waves on a SIMD (at 96 scalar registers seven fit, 6% slower).
+// 128 x 128 x 32 blocks, 128 rays, FP16 field: 5065 us with one body for every
+// ray, 4205 us now; 24 worlds in a batch 2610 -> 2324 us.
+
+// Wave-uniform loads through the scalar cache: data that no thread of this
+// launch writes, at an address that is the same for the whole wave.
+template <class T>
+__device__ __forceinline__ T scalar_load(const void* base, unsigned i) {
+    typedef uint32_t Raw __attribute__((ext_vector_type(sizeof(T) / 4)));
+    typedef const __attribute__((address_space(4))) Raw* P;
+    const Raw raw = *(P)(uintptr_t)((const char*)base + (size_t)i * sizeof(T));
+    return __builtin_bit_cast(T, raw);
+}
+// Byte i of an array, and element i of an int16 array (the dword that holds it
+// is inside the world's block, whose parts are 256-byte aligned).
+__device__ __forceinline__ unsigned scalar_u8(const uint8_t* base, unsigned i) {
+    const uintptr_t at = (uintptr_t)base + i;
+    return (scalar_load<uint1>((const void*)(at & ~(uintptr_t)3), 0).x >> ((at & 3) * 8)) & 0xffu;
+}
+__device__ __forceinline__ int scalar_i16(const int16_t* base, unsigned i) {
+    return (int)(int16_t)(scalar_load<uint1>(base, i >> 1).x >> ((i & 1) * 16));
+}
+
+// trace_ray's shading of a hit.
+__device__ __forceinline__ f3 shade_material(const WorldView& w, int voxel, f3 prop) {
+    const MatF m = get_mat(w, voxel);
+    const f3 zero = {0.0f, 0.0f, 0.0f};
+    return zero + (prop * m.color + m.color * m.emit);
+}
+
+// The refinement of refine_hit after a coarse hit in the block of grid key
+// `key` (its id `id`), for a ray in div_range and a start no lower than -8.
+// Voxels of one block in a row cost one load each: the block id is fetched
+// only when the block changes.
+__device__ __forceinline__ RayHit refine_grid(const RadianceArgs& a, const MarchRay& m, f3 bh, int key, int id) {
+    const WorldView& w = a.world;
+    const int kx = w.wx + 2, kxy = kx * (w.wy + 2);
+    const f3 d = m.d, inv = m.inv;
+    // Voxel coordinates as floats (exact integers): truncation towards zero.
+    f3 v = {truncf(bh.x), truncf(bh.y), truncf(bh.z)};
+    auto fetch = [&]() {
+        const int ix = (int)v.x, iy = (int)v.y, iz = (int)v.z;
+        // Block 0 also holds -15 .. -1 (the shader's truncating division).
+        const int bx = block_axis(ix), by = block_axis(iy), bz = block_axis(iz);
+        const int k = bx + __mul24(by, kx) + __mul24(bz, kxy);
+        if (k != key) {
+            key = k;
+            id = 0;
+            if (bx < w.wx && by < w.wy && bz < w.wz) id = block_id(w, bx, by, bz);
+            if (id >= w.palette_slots) id = 0;
+        }
+        int cv = 0;
+        if (id != 0) cv = gld(w.palette, ((uint32_t)id << 12) | voxel_offset(ix, iy, iz));
+        return cv;
+    };
+    RayHit r;
+    r.hit = 1;
+    int cv = fetch();
+    f3 st = {0.0f, 0.0f, 0.0f}, tf = st;
+    const f3 s = {__builtin_copysignf(1.0f, d.x), __builtin_copysignf(1.0f, d.y), __builtin_copysignf(1.0f, d.z)};
+    if (cv == 0) {
+        const f3 fl = {floorf(bh.x), floorf(bh.y), floorf(bh.z)};
+        const f3 q = fl - bh;
+        f3 c1 = {div_rn(q.x, d.x, inv.x), div_rn(q.y, d.y, inv.y), div_rn(q.z, d.z, inv.z)};
+        if (!div_range(bh)) c1 = {q.x / d.x, q.y / d.y, q.z / d.z};
+        const f3 c2 = c1 + inv;
+        f3 t = {fmaxf(c1.x, c2.x), fmaxf(c1.y, c2.y), fmaxf(c1.z, c2.z)};
+        const f3 dt = {fabsf(inv.x), fabsf(inv.y), fabsf(inv.z)};
+        int left = 5;
+        do {
+            // Every axis at the minimum steps (ties step together).
+            const float tm = fminf(t.x, fminf(t.y, t.z));
+            st = {t.x == tm ? 1.0f : 0.0f, t.y == tm ? 1.0f : 0.0f, t.z == tm ? 1.0f : 0.0f};
+            // Products with 0 or 1 are exact: one rounding, as t + dt * st.
+            v = {fmaf(s.x, st.x, v.x), fmaf(s.y, st.y, v.y), fmaf(s.z, st.z, v.z)};
+            t = {fmaf(dt.x, st.x, t.x), fmaf(dt.y, st.y, t.y), fmaf(dt.z, st.z, t.z)};
+            cv = fetch();
+        } while (--left > 0 && cv == 0);
+        tf = t - dt;
+    }
+    r.normal = -(s * st);
+    r.fraction = dot3(tf, st);
+    r.voxel = cv;
+    return r;
+}
+
+// cast_ray over the world's march grid, for a ray that starts in the world
+// and is at most kGridMaxDist long (so no sample lies more than one block
+// outside the world); slot 0 is air.
+//
+// The fractions of a ray's samples do not depend on what it reads as long as
+// it stays in plain air, so two samples are taken at a time: the second's grid
+// byte is on its way before the first's arrives, and counts only if the first
+// was air.  (A second sample after a first outside the world may lie further
+// out: its index is clamped.)  Grid indices are formed in floats, exact below
+// 2^24: six 2-cycle operations and a conversion instead of three conversions
+// and two 4-cycle multiply-adds.
+//
+// In a block that holds something, samples lie half a voxel apart.  The grid
+// byte tells its empty octants: n samples in one are passed by at once.
+//   - Positions: an axis is monotone in the fraction, so samples between the
+//     current one and one short of the octant's far face stay inside it.
+//     Rounding moves a position by under 2^-9 (worlds up to 512 blocks an
+//     axis), the face is taken 2^-8 early.
+//   - The fraction: adding 1/2 is exact but where the result enters the next
+//     binade, and it does so once (n + 1 samples at most double it); rounding
+//     there commutes with adding multiples of 1/2.
+// Elsewhere the next kAhead samples are loaded together: 2 take 288 us where
+// 1 takes 320 us for a world with 32 models (48 x 48 x 16 blocks, 64 rays, map
+// and glossy query included); 4 take 303 us, being past 64 registers.
+__device__ __forceinline__ RayHit cast_ray_grid(const RadianceArgs& a, f3 o, f3 d) {
+    const WorldView& w = a.world;
+    const MarchRay m = march_ray(o, d);
+    const int kx = w.wx + 2, kxy = kx * (w.wy + 2);
+    float fx = (float)kx, fxy = (float)kxy, corner = (float)(1 + kx + kxy), last = (float)(kxy * (w.wz + 2) - 1);
+    struct Sample {
+        float fraction, next;  // here, and past the block if it is air
+        float index;
+    };
+    auto sample = [&](float from) {
+        Sample q;
+        q.fraction = from + 0.5f;
+        const f3 pos = m.o + m.d * q.fraction;
+        const f3 ps = pos * 0.0625f;
+        // The truncating block coordinate for p >= 0; the padding below 0.
+        const f3 cell = {floorf(ps.x), floorf(ps.y), floorf(ps.z)};
+        q.index = fmaf(cell.y, fx, fmaf(cell.z, fxy, corner)) + cell.x;
+        const f3 box = {fmaf(cell.x, 16.0f, m.corner.x), fmaf(cell.y, 16.0f, m.corner.y),
+                        fmaf(cell.z, 16.0f, m.corner.z)};
+        const f3 tmp = (-pos) * m.inv;
+        const f3 bc = box * m.inv + tmp;
+        q.next = q.fraction + fmaxf(fminf(bc.x, fminf(bc.y, bc.z)), 0.01f);
+        return q;
+    };
+    float fraction = 0.0f;
+    constexpr int kAhead = 2;
+    constexpr float kMargin = 0.00390625f;
+    const f3 near = {d.x > 0.0f ? 8.0f - kMargin : kMargin, d.y > 0.0f ? 8.0f - kMargin : kMargin,
+                     d.z > 0.0f ? 8.0f - kMargin : kMargin};
+    int left = a.max_steps > 0 ? a.max_steps : 1 << 20;  // samples
+    int state = 0, id = 0, key = 0;
+    while (state == 0) {
+        bool air;
+        unsigned mask;
+        do {
+            const Sample s0 = sample(fraction);
+            const uint8_t b0 = gld(a.grid, (unsigned)s0.index);
+            const Sample s1 = sample(s0.next);
+            const uint8_t b1 = gld(a.grid, (unsigned)fminf(s1.index, last));
+            bool second = b0 == 0 && s0.next < a.max_dist;
+            if (a.max_steps > 0) {
+                second = second && left > 1;
+                left -= second ? 2 : 1;
+            }
+            mask = second ? b1 : b0;
+            air = mask == 0;
+            fraction = second ? s1.fraction : s0.fraction;
+            if (air) {
+                fraction = second ? s1.next : s0.next;
+                if (fraction >= a.max_dist || (a.max_steps > 0 && left == 0)) state = -1;
+            }
+        } while (air && state == 0);
+        if (!air) {
+            // A block that is not empty, or a sample outside the world, in
+            // coarse_sample's order of tests; then the samples half a voxel
+            // apart that stay in that block.
+            f3 pos = m.o + m.d * fraction;
+            int ix = (int)pos.x, iy = (int)pos.y, iz = (int)pos.z;
+            const int bx = block_axis(ix), by = block_axis(iy), bz = block_axis(iz);
+            id = 0;
+            if (block_axis_in(ix, w.wx) && block_axis_in(iy, w.wy) && block_axis_in(iz, w.wz))
+                id = block_id(w, bx, by, bz);
+            if (mask == 0xffu && id == 0) state = -1;  // outside, or air below 0
+            const uint32_t slot = (uint32_t)id << 12;
+            const bool voxels = (unsigned)(id - 1) < (unsigned)(w.palette_slots - 1);
+            auto leaves = [&]() {
+                return fminf(pos.x, fminf(pos.y, pos.z)) < 0.0f || fraction >= a.max_dist || left == 0;
+            };
+            key = bx + __mul24(by, kx) + __mul24(bz, kxy);
+            if (voxels && gld(w.palette, slot | voxel_offset(ix, iy, iz)) != 0) state = 1;
+            else if (leaves()) state = -1;
+            bool same = true;
+            while (state == 0 && same) {
+                const unsigned oct = ((ix >> 3) & 1) | ((iy >> 2) & 2) | ((iz >> 1) & 4);
+                if (!((mask >> oct) & 1)) {
+                    // Straight on to the last sample in this empty octant.
+                    const f3 end = {(float)(ix & ~7) + near.x, (float)(iy & ~7) + near.y, (float)(iz & ~7) + near.z};
+                    const f3 t = (end - m.o) * m.inv;
+                    const float stop = fminf(fminf(t.x, fminf(t.y, t.z)), fminf(a.max_dist, 2.0f * fraction) - 0.5f);
+                    const float n = fminf(truncf((stop - fraction) * 2.0f), (float)(left - 1));
+                    if (n > 0.0f) {
+                        fraction = fmaf(n, 0.5f, fraction);
+                        left -= (int)n;
+                    }
+                }
+                // The next kAhead samples at once.
+                float f[kAhead];
+                f3 p[kAhead];
+                int q[3][kAhead];
+                uint8_t v[kAhead];
+#pragma unroll
+                for (int k = 0; k < kAhead; ++k) {
+                    f[k] = (k ? f[k - 1] : fraction) + 0.5f;
+                    p[k] = m.o + m.d * f[k];
+                    q[0][k] = (int)p[k].x;
+                    q[1][k] = (int)p[k].y;
+                    q[2][k] = (int)p[k].z;
+                    v[k] = 0;
+                    if (voxels) v[k] = gld(w.palette, slot | voxel_offset(q[0][k], q[1][k], q[2][k]));
+                }
+#pragma unroll
+                for (int k = 0; k < kAhead; ++k) {
+                    same = same && (unsigned)((q[0][k] ^ ix) | (q[1][k] ^ iy) | (q[2][k] ^ iz)) < 16u;
+                    if (state == 0 && same) {  // else the grid takes it from the last sample in the block
+                        fraction = f[k];
+                        pos = p[k];
+                        --left;
+                        if (v[k] != 0) state = 1;
+                        else if (leaves()) state = -1;
+                    }
+                }
+                ix = (int)pos.x;
+                iy = (int)pos.y;
+                iz = (int)pos.z;
+            }
+        }
+    }
+    RayHit h;
+    h.hit = 0;
+    if (state > 0) {
+        const f3 bh = m.o + m.d * (fraction - 1.5f);
+        if (div_range(m.d) && fminf(bh.x, fminf(bh.y, bh.z)) >= -8.0f) h = refine_grid(a, m, bh, key, id);
+        else h = refine_hit(w, m, fraction);
+    }
+    return h;
+}
+
+// Raw components of hash33 (32-bit integers), on the scalar unit for a
+// uniform key.
+__device__ __forceinline__ uint3 hash33_raw(uint32_t x, uint32_t t) {
+    const uint32_t k = 1103515245u;
+    uint32_t y = t, z = t;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const uint32_t nx = ((x >> 8) ^ y) * k, ny = ((y >> 8) ^ z) * k, nz = ((z >> 8) ^ x) * k;
+        x = nx;
+        y = ny;
+        z = nz;
+    }
+    return make_uint3(x, y, z);
+}
+
+// v of the next lane; `last` for lane 63.
+__device__ __forceinline__ float from_next_lane(float v, float last) {
+    constexpr int kWaveShl1 = 0x130;
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(last), __float_as_int(v), kWaveShl1, 0xF, 0xF, false));
+}
+
+// ray_setup of rays key * R + r0 + lane of one probe, for a whole wave.
+__device__ __forceinline__ void chunk_rays(uint32_t t, uint32_t first, float4 fb, uint32_t flip, int px, int py,
+                                           int pz, f3* pos_out, f3* dir_out) {
+    const uint3 h = hash33_raw(first + (threadIdx.x & 63), t), e = hash33_raw(first + 64u, t);
+    const f3 h0 = {(float)h.x, (float)h.y, (float)h.z};
+    const f3 h1 = {from_next_lane(h0.x, (float)e.x), from_next_lane(h0.y, (float)e.y), from_next_lane(h0.z, (float)e.z)};
+    // (hash33 - 0.5) * 2 = RN(h - 2^31) * 2^-31; powers of two move through every rounding.
+    const f3 c31 = {2147483648.0f, 2147483648.0f, 2147483648.0f};
+    const f3 center = {(float)(px * 16 + 8), (float)(py * 16 + 8), (float)(pz * 16 + 8)};
+    f3 dir = normalize3_near1(f3{fb.x, fb.y, fb.z} + (0.1f * 0x1p-31f) * (h0 - c31));
+    f3 pos = center + dir * 6.0f;
+    const f3 j1 = h1 - c31;
+    pos = {fmaf(j1.x, 0x1p-31f, pos.x), fmaf(j1.y, 0x1p-31f, pos.y), fmaf(j1.z, 0x1p-31f, pos.z)};
+    *pos_out = pos;
+    *dir_out = {__uint_as_float(__float_as_uint(dir.x) ^ flip), __uint_as_float(__float_as_uint(dir.y) ^ flip),
+                __uint_as_float(__float_as_uint(dir.z) ^ flip)};
+}
+
+// Whether the ray from o along d ends in its own block (px, py, pz), slot
+// `blk`, without a step; then its voxel.
+__device__ __forceinline__ bool ends_inside(const WorldView& w, int blk, f3 o, f3 d, int px, int py, int pz, int* voxel) {
+    const f3 p0 = {fmaf(d.x, 0.5f, o.x), fmaf(d.y, 0.5f, o.y), fmaf(d.z, 0.5f, o.z)};  // fraction 0.5 (d / 2 is exact)
+    const f3 p1 = o - d;                                                              // fraction 0.5 - 1.5
+    const uint8_t* slot = w.palette + ((size_t)blk << 12);
+    const int v0 = gld(slot, voxel_offset((int)p0.x, (int)p0.y, (int)p0.z));
+    const unsigned lx = (unsigned)((int)p1.x - px * 16), ly = (unsigned)((int)p1.y - py * 16),
+                   lz = (unsigned)((int)p1.z - pz * 16);
+    bool inside = false;
+    if ((lx | ly | lz) < 16u) {
+        const int v1 = gld(slot, lx + (ly << 4) + (lz << 8));
+        *voxel = v1;
+        // Axis-parallel rays take the general path (their fraction can be NaN).
+        inside = v0 != 0 && v1 != 0 && fminf(fminf(fabsf(d.x), fabsf(d.y)), fabsf(d.z)) >= kTiny;
+    }
+    return inside;
+}
+
+// Octant of the escape masks a direction points into.
+__device__ __forceinline__ unsigned escape_octant(f3 d) {
+    return (__float_as_uint(d.x) >> 31) | ((__float_as_uint(d.y) >> 31) << 1) | ((__float_as_uint(d.z) >> 31) << 2);
+}
+
+// UNI: R >= 64, a wave's rays belong to one probe.  tid as for
+// radiance_lane_body.
+template <int STORE, bool UNI>
+__device__ __forceinline__ void radiance_chunk_body(const RadianceArgs& a, const int time_seed, const int tid, f3* chunk_sum) {
+    const WorldView& w = a.world;
+    const int R = a.rays, lane = threadIdx.x & 63;
+    int wg, k = 0, r;  // probe, chunk of the probe, ray of the probe
+    if constexpr (UNI) {
+        const int c = __builtin_amdgcn_readfirstlane(tid >> 6), per = R >> 6;
+        wg = a.log2_rays >= 0 ? c >> (a.log2_rays - 6) : c / per;
+        k = c - wg * per;
+        r = k * 64 + lane;
+    } else {
+        wg = tid >> a.log2_rays;
+        r = tid & (R - 1);
+    }
+    int x = 0, y = 0, z = 0, key = wg;
+    const bool valid = probe_coords(a, wg, &x, &y, &z, &key);
+    f3 light = {0.0f, 0.0f, 0.0f};
+    if (valid) {
+        f3 o, d;
+        int blk;
+        unsigned escape = 0;
+        if constexpr (UNI) {
+            x = __builtin_amdgcn_readfirstlane(x);
+            y = __builtin_amdgcn_readfirstlane(y);
+            z = __builtin_amdgcn_readfirstlane(z);
+            key = __builtin_amdgcn_readfirstlane(key);
+            const unsigned block = (unsigned)x + (unsigned)w.wx * ((unsigned)y + (unsigned)w.wy * (unsigned)z);
+            blk = scalar_i16(w.blocks, block);
+            if (a.grid) escape = scalar_u8(a.escape, block);
+            const uint32_t first = (uint32_t)key * (uint32_t)R + (uint32_t)k * 64u + (uint32_t)time_seed;
+            chunk_rays((uint32_t)time_seed, first, gld(a.fib, (size_t)r), (uint32_t)lane << 31, x, y, z, &o, &d);
+        } else {
+            const unsigned block = (unsigned)x + mul24((unsigned)w.wx, (unsigned)y + mul24((unsigned)w.wy, (unsigned)z));
+            blk = gld(w.blocks, block);
+            if (a.grid) escape = gld(a.escape, block);
+            ray_setup(a, time_seed, key, r, x, y, z, &o, &d);
+        }
+        bool march = true;
+        if (blk == 0) {
+            if ((escape >> escape_octant(d)) & 1) {
+                light = sky_light(d);
+                march = false;
+            }
+        } else if ((unsigned)blk < (unsigned)w.palette_slots) {
+            int voxel = 0;
+            if (ends_inside(w, blk, o, d, x, y, z, &voxel)) {
+                // o / 16 - cell: o / 16 is exact.
+                const f3 t = {fmaf(o.x, 0.0625f, -(float)x), fmaf(o.y, 0.0625f, -(float)y), fmaf(o.z, 0.0625f, -(float)z)};
+                f3 prop;
+                if constexpr (UNI) {
+                    const unsigned x1 = x + 1 == w.wx ? 0 : x + 1, y1 = y + 1 == w.wy ? 0 : y + 1,
+                                   z1 = z + 1 == w.wz ? 0 : z + 1;
+                    const unsigned r00 = w.wx * (y + w.wy * z), r10 = w.wx * (y1 + w.wy * z);
+                    const unsigned r01 = w.wx * (y + w.wy * z1), r11 = w.wx * (y1 + w.wy * z1);
+                    auto texel = [&](unsigned i) {
+                        return Texel<STORE>::unpack(scalar_load<typename Texel<STORE>::type>(a.field_in, i));
+                    };
+                    prop = trilinear(texel(r00 + x), texel(r00 + x1), texel(r10 + x), texel(r10 + x1), texel(r01 + x),
+                                     texel(r01 + x1), texel(r11 + x), texel(r11 + x1), t);
+                } else {
+                    prop = sample_taps<STORE>(a.field_in, w.wx, w.wy, w.wz, x, y, z, t);
+                }
+                light = shade_material(w, voxel, prop);
+                march = false;
+            }
+        }
+        if (march) {
+            RayHit h;
+            if (a.grid) h = cast_ray_grid(a, o, d);
+            else h = cast_ray(w, o, d, a.max_dist, a.max_steps);
+            if (h.hit)
+                light = shade_material(w, h.voxel, sample_radiance<STORE>(a.field_in, w.wx, w.wy, w.wz,
+                                                                          o + h.fraction * d, h.normal));
+            else
+                light = sky_light(d);
+        }
+    }
+    f3 sum = butterfly(light, UNI ? 64 : R);
+    if constexpr (UNI) {
+        if (R > 64) {  // chunk sums in chunk order; a probe's waves share a workgroup
+            const int wave = threadIdx.x >> 6;
+            if (lane == 0) chunk_sum[wave] = sum;
+            __syncthreads();
+            if (r == 0)
+                for (int c = 1; c < R >> 6; ++c) sum = sum + chunk_sum[wave + c];
+        }
+    }
+    if (valid && r == 0) store_probe<STORE>(a, wg, x, y, z, sum);
+}
+
+template <int STORE, bool UNI>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8))) radiance_chunk_kernel(RadianceArgs a) {
+    extern __shared__ f3 chunk_sum[];
+    radiance_chunk_body<STORE, UNI>(a, a.time_seed, (int)(blockIdx.x * blockDim.x + threadIdx.x), chunk_sum);
+}
+
 template <int STORE, bool TRACED, bool OCC, int K>
 __global__ void __launch_bounds__(1024) radiance_kernel(RadianceArgs a) {
     extern __shared__ f3 chunk_sum[];
-    radiance_lane_body<STORE, TRACED, OCC, K>(a, blockIdx.x * blockDim.x + threadIdx.x, chunk_sum);
+    radiance_lane_body<STORE, TRACED, OCC, K>(a, a.time_seed, blockIdx.x * blockDim.x + threadIdx.x, chunk_sum);
 }
 
 // Lane refill (tuning variant 3; 64 rays per probe).  A wave owns probes
@@ -350,7 +763,7 @@ __global__ void __launch_bounds__(256) radiance_refill_kernel(RadianceArgs a, in
         f3 pos = {-64.0f, -64.0f, -64.0f}, dir = {0.57735027f, 0.57735027f, 0.57735027f};
         // A probe not dispatched or outside the world marches from outside it
         // and leaves at its first sample; its light is not used.
-        if (probe_coords(a, wg0 + j, &px, &py, &pz, &key)) ray_setup(a, key, lane, px, py, pz, &pos, &dir);
+        if (probe_coords(a, wg0 + j, &px, &py, &pz, &key)) ray_setup(a, a.time_seed, key, lane, px, py, pz, &pos, &dir);
         const MarchRay m = march_ray(pos, dir);
         float* r = rs + (j * 64 + lane) * kRefillFloats;
         r[0] = m.o.x; r[1] = m.o.y; r[2] = m.o.z;
@@ -451,20 +864,31 @@ hipError_t launch_radiance_refill(const RadianceArgs& a, int store, int P, hipSt
 // SERVED only separates the serving engine's launches from the batch API's
 // in profiles; the code is the same.
 template <int STORE, bool OCC, bool SERVED, int K>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8)))
 radiance_batch_kernel(const RadianceArgs* args, const int* begin, int n_worlds, const int* frame) {
     extern __shared__ f3 chunk_sum[];
     const int b0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * blockDim.x));
-    int lo = 0, hi = n_worlds - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (begin[mid] <= b0) lo = mid;
-        else hi = mid - 1;
+    // The last world that begins at or before b0: 64 worlds a step, one a lane
+    // (a scalar binary search is a chain of loads, 1% of the launch).
+    int lo = -1;
+    for (int w0 = 0; w0 < n_worlds; w0 += 64) {
+        const int i = w0 + (int)(threadIdx.x & 63);
+        const int in = __popcll(__ballot(i < n_worlds && begin[i] <= b0));
+        lo += in;
+        if (in < 64) break;
     }
-    lo = __builtin_amdgcn_readfirstlane(lo);
-    RadianceArgs a = args[lo];
-    if (frame) a.time_seed += *frame;
-    radiance_lane_body<STORE, false, OCC, K>(a, (int)(blockIdx.x * blockDim.x + threadIdx.x) - begin[lo], chunk_sum);
+    // Arguments as constants (no thread writes them): each is loaded where it
+    // is used and takes no register before.  A copy held 106 scalar registers,
+    // six waves a SIMD: 2672 us for 24 worlds, 2389 us without it.
+    const RadianceArgs& a = *(const RadianceArgs*)(const __attribute__((address_space(4))) RadianceArgs*)(uintptr_t)(args + lo);
+    const int time_seed = a.time_seed + (frame ? *frame : 0);
+    const int tid = (int)(blockIdx.x * blockDim.x + threadIdx.x) - begin[lo];
+    if constexpr (K == 1 && !OCC) {
+        if (a.rays >= 64) radiance_chunk_body<STORE, true>(a, time_seed, tid, chunk_sum);
+        else radiance_chunk_body<STORE, false>(a, time_seed, tid, chunk_sum);
+    } else {
+        radiance_lane_body<STORE, false, OCC, K>(a, time_seed, tid, chunk_sum);
+    }
 }
 
 template <int STORE, bool SERVED>
@@ -508,6 +932,13 @@ static hipError_t launch_store(const RadianceArgs& a, hipStream_t stream) {
     int grid = (int)((threads + bs - 1) / bs);
     size_t lds = sizeof(f3) * (bs / 64) * K;
     if (grid == 0) return hipSuccess;
+    if constexpr (K == 1 && !TRACED && !OCC) {
+        if (R >= 64)
+            hipLaunchKernelGGL((radiance_chunk_kernel<STORE, true>), dim3(grid), dim3(bs), lds, stream, a);
+        else
+            hipLaunchKernelGGL((radiance_chunk_kernel<STORE, false>), dim3(grid), dim3(bs), lds, stream, a);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL((radiance_kernel<STORE, TRACED, OCC, K>), dim3(grid), dim3(bs), lds, stream, a);
     return hipGetLastError();
 }
@@ -976,7 +1407,7 @@ __global__ void __launch_bounds__(1024) radiance_tiled_kernel(RadianceArgs a) {
             }
             if (valid) {
                 f3 pos, dir;
-                ray_setup(a, wg, l, px, py, pz, &pos, &dir);
+                ray_setup(a, a.time_seed, wg, l, px, py, pz, &pos, &dir);
                 RayHit h = cast_ray_occ(occ, pos, dir, a.max_dist, a.max_steps);
                 if (h.hit) {
                     const float* m = s_mats + h.voxel * 6;
@@ -1128,7 +1559,8 @@ __global__ void __launch_bounds__(256) block_bits_kernel(const int16_t* blocks, 
 
 // Per-slot voxel-occupancy bits: one workgroup of 128 threads per slot, one
 // output word (32 voxels) per thread.
-__global__ void __launch_bounds__(128) palette_bits_kernel(const uint8_t* palette, int first, uint32_t* bits) {
+__global__ void __launch_bounds__(128) palette_bits_kernel(const uint8_t* palette, int first, uint32_t* bits,
+                                                           uint8_t* slot_mask, int fill_end) {
     const int slot = first + blockIdx.x;
     const uint8_t* src = palette + ((size_t)slot << 12) + threadIdx.x * 32;
     const uint4 a0 = ((const uint4*)src)[0];
@@ -1138,6 +1570,9 @@ __global__ void __launch_bounds__(128) palette_bits_kernel(const uint8_t* palett
 #pragma unroll
     for (int k = 0; k < 32; ++k) v |= (((w[k >> 2] >> ((k & 3) * 8)) & 0xffu) != 0 ? 1u : 0u) << k;
     bits[((size_t)slot << 7) + threadIdx.x] = v;
+    if (slot_mask) slot_octants(v, slot, slot_mask);
+    const int n = (int)gridDim.x;
+    for (int i = first + n + (int)(blockIdx.x * 128 + threadIdx.x); i < fill_end; i += n * 128) slot_mask[i] = 0xff;
 }
 
 hipError_t launch_block_bits(const int16_t* blocks, int n_blocks, uint32_t* bits, hipStream_t stream) {
@@ -1147,10 +1582,152 @@ hipError_t launch_block_bits(const int16_t* blocks, int n_blocks, uint32_t* bits
     return hipGetLastError();
 }
 
+// March grid of a world (lumx_internal.hpp, MarchGrid) from its empty-block
+// bits and its slots' octants.  A workgroup takes 32 x 4 x 4 blocks: the rows
+// of the tile and of the 8 blocks around it as 64-bit words of "not empty"
+// bits (bit 8 is the tile's first block), windowed along x with shifts, then
+// along y and z by ORing nine rows of LDS.
+constexpr int kGridTileX = 32, kGridTileY = 4, kGridTileZ = 4, kGridReach = 8;
+constexpr int kGridRows = kGridTileY + 2 * kGridReach;  // rows per axis of the haloed tile
+typedef unsigned long long u64;
+struct GridLds {
+    u64 pos[kGridRows * kGridRows];  // [z][y]: windows towards +x and -x
+    u64 neg[kGridRows * kGridRows];
+    u64 wy[4][kGridRows][kGridTileY];  // [sign x + 2 sign y][z][tile y]
+    uint32_t free[8][kGridTileZ][kGridTileY];  // per octant: bit x of a tile row
+};
+
+__device__ __forceinline__ void march_grid_tile(const GridArgs& g, int tile, GridLds& lds) {
+    static_assert(kGridTileY == kGridTileZ, "the haloed tile is square in y and z");
+    const int tx = (g.wx + kGridTileX - 1) / kGridTileX, ty = (g.wy + kGridTileY - 1) / kGridTileY;
+    const int x0 = (tile % tx) * kGridTileX, y0 = (tile / tx % ty) * kGridTileY, z0 = tile / (tx * ty) * kGridTileZ;
+    const int T = blockDim.x, tid = threadIdx.x;
+    // Blocks x0 - 8 .. x0 + 39 of a row, clipped to the world.
+    const int xs = max(x0 - kGridReach, 0), xe = min(x0 + kGridTileX + kGridReach, g.wx);
+    for (int i = tid; i < kGridRows * kGridRows; i += T) {
+        const int y = y0 - kGridReach + i % kGridRows, z = z0 - kGridReach + i / kGridRows;
+        u64 v = 0;
+        if ((unsigned)y < (unsigned)g.wy && (unsigned)z < (unsigned)g.wz) {
+            const unsigned bit = (unsigned)xs + (unsigned)g.wx * ((unsigned)y + (unsigned)g.wy * (unsigned)z);
+            const unsigned last = ((unsigned)g.n_blocks - 1) >> 5, k = bit >> 5;
+            const u64 lo = g.empty_bits[k] | ((u64)g.empty_bits[min(k + 1, last)] << 32);
+            const u64 hi = g.empty_bits[min(k + 2, last)];
+            const int sh = bit & 31;
+            v = lo >> sh;
+            if (sh) v |= hi << (64 - sh);
+            v = (~v & ((1ull << (xe - xs)) - 1)) << (xs - (x0 - kGridReach));
+        }
+        u64 p = v | (v >> 1), n = v | (v << 1);  // windows of 9 blocks
+        p |= p >> 2;
+        n |= n << 2;
+        p |= p >> 4;
+        n |= n << 4;
+        lds.pos[i] = p | (v >> 8);
+        lds.neg[i] = n | (v << 8);
+    }
+    // The grid bytes of the tile and of the padding next to it.
+    constexpr int kPadX = kGridTileX + 2, kPadY = kGridTileY + 2, kPadZ = kGridTileZ + 2;
+    for (int i = tid; i < kPadX * kPadY * kPadZ; i += T) {
+        const int x = x0 - 1 + i % kPadX, y = y0 - 1 + i / kPadX % kPadY, z = z0 - 1 + i / (kPadX * kPadY);
+        if (x > g.wx || y > g.wy || z > g.wz) continue;
+        // Outside the tile: padding only, by the tile that its nearest block is in.
+        const int cx = min(max(x, 0), g.wx - 1), cy = min(max(y, 0), g.wy - 1), cz = min(max(z, 0), g.wz - 1);
+        if ((unsigned)(cx - x0) >= kGridTileX || (unsigned)(cy - y0) >= kGridTileY || (unsigned)(cz - z0) >= kGridTileZ)
+            continue;
+        unsigned byte = 0xffu;
+        if (cx == x && cy == y && cz == z) {
+            const int id = g.blocks[(unsigned)x + (unsigned)g.wx * ((unsigned)y + (unsigned)g.wy * (unsigned)z)];
+            byte = id == 0 ? 0u : g.slot_mask && (unsigned)id < (unsigned)g.slots ? max(g.slot_mask[id], (uint8_t)1) : 0xffu;
+        }
+        g.grid[(unsigned)(x + 1) + (unsigned)(g.wx + 2) * ((unsigned)(y + 1) + (unsigned)(g.wy + 2) * (unsigned)(z + 1))] =
+            (uint8_t)byte;
+    }
+    __syncthreads();
+    for (int i = tid; i < 4 * kGridRows * kGridTileY; i += T) {
+        const int y = i % kGridTileY, z = i / kGridTileY % kGridRows, c = i / (kGridTileY * kGridRows);
+        const u64* row = (c & 1 ? lds.pos : lds.neg) + z * kGridRows + y + kGridReach;
+        const int step = c & 2 ? 1 : -1;
+        u64 v = 0;
+#pragma unroll
+        for (int k = 0; k <= kGridReach; ++k) v |= row[k * step];
+        lds.wy[c][z][y] = v;
+    }
+    __syncthreads();
+    for (int i = tid; i < 8 * kGridTileY * kGridTileZ; i += T) {
+        const int y = i % kGridTileY, z = i / kGridTileY % kGridTileZ, oct = i / (kGridTileY * kGridTileZ);
+        const int step = oct & 4 ? 1 : -1;
+        u64 v = 0;
+#pragma unroll
+        for (int k = 0; k <= kGridReach; ++k) v |= lds.wy[oct & 3][z + kGridReach + k * step][y];
+        lds.free[oct ^ 7][z][y] = (uint32_t)(~v >> kGridReach);
+    }
+    __syncthreads();
+    // Thread = block: the tile's rows are consecutive x.
+    for (int i = tid; i < kGridTileX * kGridTileY * kGridTileZ; i += T) {
+        const int lx = i % kGridTileX, ly = i / kGridTileX % kGridTileY, lz = i / (kGridTileX * kGridTileY);
+        const int x = x0 + lx, y = y0 + ly, z = z0 + lz;
+        if (x >= g.wx || y >= g.wy || z >= g.wz) continue;
+        unsigned e = 0;
+#pragma unroll
+        for (int oct = 0; oct < 8; ++oct) e |= ((lds.free[oct][lz][ly] >> lx) & 1u) << oct;
+        g.escape[(unsigned)x + (unsigned)g.wx * ((unsigned)y + (unsigned)g.wy * (unsigned)z)] = (uint8_t)e;
+    }
+}
+
+__global__ void __launch_bounds__(256) march_grid_kernel(GridArgs g) {
+    __shared__ GridLds lds;
+    march_grid_tile(g, (int)blockIdx.x, lds);
+}
+
+int march_grid_tiles(int wx, int wy, int wz) {
+    return ((wx + kGridTileX - 1) / kGridTileX) * ((wy + kGridTileY - 1) / kGridTileY) *
+           ((wz + kGridTileZ - 1) / kGridTileZ);
+}
+
+hipError_t launch_march_grid(const GridArgs& g, hipStream_t stream) {
+    if (!g.grid) return hipSuccess;
+    hipLaunchKernelGGL(march_grid_kernel, dim3(g.tiles), dim3(256), 0, stream, g);
+    return hipGetLastError();
+}
+
+struct GridBatch {
+    GridArgs g[kGridBatch];
+    int begin[kGridBatch + 1];  // first workgroup of each world
+    int n;
+};
+static_assert(sizeof(GridBatch) <= 4096, "kernel arguments are limited to 4 KiB");
+
+__global__ void __launch_bounds__(256) march_grid_batch_kernel(GridBatch b) {
+    __shared__ GridLds lds;
+    int i = 0;
+    while (i + 1 < b.n && b.begin[i + 1] <= (int)blockIdx.x) ++i;
+    march_grid_tile(b.g[i], (int)blockIdx.x - b.begin[i], lds);
+}
+
+hipError_t launch_march_grid_batch(const GridArgs* g, int n, hipStream_t stream) {
+    for (int i = 0; i < n;) {
+        GridBatch b{};
+        while (i < n && b.n < kGridBatch && (b.n == 0 || b.begin[b.n] < (1 << 24))) {
+            if (g[i].grid) {
+                b.g[b.n] = g[i];
+                b.begin[b.n + 1] = b.begin[b.n] + g[i].tiles;
+                ++b.n;
+            }
+            ++i;
+        }
+        if (!b.n) continue;
+        hipLaunchKernelGGL(march_grid_batch_kernel, dim3(b.begin[b.n]), dim3(256), 0, stream, b);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 hipError_t launch_palette_bits(const uint8_t* palette, int first_slot, int n_slots, uint32_t* bits,
-                               hipStream_t stream) {
+                               uint8_t* slot_mask, int fill_end, hipStream_t stream) {
     if (n_slots <= 0) return hipSuccess;
-    hipLaunchKernelGGL(palette_bits_kernel, dim3(n_slots), dim3(128), 0, stream, palette, first_slot, bits);
+    hipLaunchKernelGGL(palette_bits_kernel, dim3(n_slots), dim3(128), 0, stream, palette, first_slot, bits, slot_mask,
+                       fill_end);
     return hipGetLastError();
 }
 

@@ -31,6 +31,28 @@ __device__ __forceinline__ void attach_world(const AttachArgs& a, long long firs
         a.blockify_state[2] = 0;
         a.blockify_state[3] = 0;
     }
+    // Eight lanes a slot, one octant each (first is a thread's number and the
+    // stride a multiple of 64, so the lanes of a slot sit side by side).
+    const long long n_oct = a.slot_mask ? (long long)a.slots * 8 : 0;
+    for (long long i = first; i < n_oct; i += stride) {
+        const int slot = (int)(i >> 3), oct = (int)(i & 7);
+        bool any = false;
+        if (slot < a.used) {
+            const uint8_t* src = a.palette + ((size_t)slot << 12) + ((oct & 1) << 3) + ((oct & 2) << 6) + ((oct & 4) << 9);
+            uint2 v = make_uint2(0u, 0u);
+            for (int z = 0; z < 8; ++z) {
+#pragma unroll
+                for (int y = 0; y < 8; ++y) {
+                    const uint2 r = *(const uint2*)(src + z * 256 + y * 16);
+                    v.x |= r.x;
+                    v.y |= r.y;
+                }
+            }
+            any = (v.x | v.y) != 0;
+        }
+        const unsigned long long b = __ballot(any);
+        if (oct == 0) a.slot_mask[slot] = (uint8_t)(b >> (threadIdx.x & 56));
+    }
     for (long long i = first; i < total; i += stride) {
         long long j = i;
         if (j < n_field) {
@@ -44,7 +66,6 @@ __device__ __forceinline__ void attach_world(const AttachArgs& a, long long firs
         }
         j -= n_pal;
         if (j < n_claim) {
-            a.sel_claim[j] = a.claim_idle;
             a.upd_claim[j] = -1;
             continue;
         }
