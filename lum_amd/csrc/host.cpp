@@ -1827,6 +1827,9 @@ int lumx_select_probes(lumx_world_t w, const int32_t* special, int n_special, in
 
 // ---- glossy ----
 extern "C++" {
+// 1 / d where pixel coordinates over d are in the range of div_rn, else 0.
+static float frame_reciprocal(float d) { return d >= 1.0f && d <= 65536.0f ? 1.0f / d : 0.0f; }
+
 void lumx::glossy_args(lumx_world* w, const uint8_t* matnorm, const float* depth, int width, int height,
                        const lumx_camera* cam, float max_dist, int max_steps, float* out, int32_t* keys,
                        GlossyArgs* ap) {
@@ -1849,8 +1852,11 @@ void lumx::glossy_args(lumx_world* w, const uint8_t* matnorm, const float* depth
     }
     a.frame_w = cam->frame_size[0];
     a.frame_h = cam->frame_size[1];
+    a.inv_w = frame_reciprocal(a.frame_w);
+    a.inv_h = frame_reciprocal(a.frame_h);
     a.max_dist = max_dist;
     a.max_steps = max_steps;
+    if (w->block0_empty && max_dist <= kGlossyGridMaxDist) a.grid = w->grid;
 }
 }  // extern "C++"
 

@@ -69,6 +69,9 @@ struct RadianceArgs {
 //           voxels from the centre, so blocks at most 8 away, and rounding
 //           keeps every coordinate monotone along the ray.
 constexpr float kGridMaxDist = 128.0f;
+// Glossy rays have no escape masks, only the grid; up to this length the
+// march's margin covers the rounding of fractions.
+constexpr float kGlossyGridMaxDist = 1024.0f;
 struct GridArgs {
     const uint32_t* empty_bits;
     const int16_t* blocks;
@@ -153,8 +156,10 @@ struct GlossyArgs {
     int width, height;
     float campos[3], camdir[3], horiz[3], verti[3], light[3];
     float frame_w, frame_h;
+    float inv_w, inv_h;          // 1 / frame size (0: divide instead)
     float max_dist;
     int max_steps;
+    const uint8_t* grid;         // march grid of the world (nullptr: not available)
 };
 
 struct DiffuseArgs {

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from lum_amd import synth
-from lum_amd.api import Batch, Model, World, placement, radiance_params
+from lum_amd.api import Batch, Model, World, camera_default, placement, radiance_params
 from lum_amd._lib import RADIANCE_BF16, RADIANCE_F16, RADIANCE_F32
 
 pytestmark = pytest.mark.gpu
@@ -116,4 +116,40 @@ def test_grid_follows_blocks_palette_maps_and_residency(gpu_ctx):
         batch.close()
         for m in models:
             m.close()
+        w.close()
+
+
+@pytest.mark.parametrize("size,fmt,width,height,max_dist,max_steps", [
+    ((24, 20, 12), RADIANCE_F32, 97, 61, 128.0, 0),
+    ((24, 20, 12), RADIANCE_F16, 33, 17, 1024.0, 64),
+    ((24, 20, 12), RADIANCE_F16, 33, 17, 1025.0, 64),  # the general march
+    ((5, 5, 3), RADIANCE_BF16, 16, 16, 0.25, 1),
+    ((1, 1, 1), RADIANCE_F32, 1, 1, 128.0, 0),
+])
+def test_glossy_grid_march_bit_exact(gpu_ctx, size, fmt, width, height, max_dist, max_steps):
+    """Origins in, around and far outside the world; NaN and infinite depths;
+    unnormalized view directions on both sides of the grid's limit."""
+    import torch
+    rng = np.random.default_rng([width, *size])
+    w = make_world(gpu_ctx, size, rng, fmt, sparse_palette(rng, 32), 0.1)
+    try:
+        matnorm = rng.integers(0, 256, (height, width, 4)).astype(np.uint8)
+        depth = rng.uniform(-0.1, 0.4, (height, width)).astype(np.float32)
+        odd = rng.random((height, width))
+        depth[odd < 0.02] = np.nan
+        depth[(odd >= 0.02) & (odd < 0.04)] = np.inf
+        depth[(odd >= 0.04) & (odd < 0.06)] = -1e30
+        mn, dp = torch.from_numpy(matnorm).cuda(), torch.from_numpy(depth).cuda()
+        for scale in (1.0, 7.0, 40.0):
+            cam = camera_default(width, height)
+            for k in range(3):
+                cam.campos[k] = 8.0 * size[k]
+                cam.camdir[k] *= scale
+            for frame in ((float(width), float(height)), (0.5, 3e5)):
+                cam.frame_size[0], cam.frame_size[1] = frame
+                got = w.glossy(mn, dp, cam, max_dist, max_steps)
+                ref, _ = w.glossy(mn, dp, cam, max_dist, max_steps, traced=True)
+                torch.cuda.synchronize()
+                assert np.array_equal(got.cpu().numpy().view(np.uint32), ref.cpu().numpy().view(np.uint32))
+    finally:
         w.close()
