@@ -1315,6 +1315,7 @@ static int map_device(lumx_world_t w, int n, const lumx_model_t* models, const l
     a.blocks = w->blocks;
     a.copy_src = w->copy_src_dev;
     a.palette = w->palette;
+    a.empty_bits = w->empty_bits;
     a.claim = w->block_claim;
     a.n_blocks = w->n_blocks;
     a.wx = w->desc.size[0];
@@ -1335,7 +1336,6 @@ static int map_device(lumx_world_t w, int n, const lumx_model_t* models, const l
     const int prev_bound = w->host_stale ? w->dev_counter_bound : std::max(w->counter, w->prev_counter);
     const int bound = (int)std::min<long long>(slots, std::max<long long>(st + total, prev_bound));
     HIP_TRY(launch_blockify(a, bound - st, s));
-    HIP_TRY(launch_block_bits(w->blocks, w->n_blocks, w->empty_bits, s));
     int rc = launch_models(w, n, models, pl, s);
     if (rc) return rc;
     // The claims took the place of every slot's mask.

@@ -206,6 +206,7 @@ struct BlockifyArgs {
     int16_t* blocks;            // current world
     int32_t* copy_src;          // per slot: static source block
     uint8_t* palette;
+    uint32_t* empty_bits;       // per block: 1 = id 0
     int* claim;                 // per block: first model covering it (this map's scratch)
     int n_blocks;
     int wx, wy, wz;

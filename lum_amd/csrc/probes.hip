@@ -29,13 +29,17 @@
 #include <stdint.h>
 
 #include "lumx_internal.hpp"
+#include "scan.hpp"
 
 namespace lumx {
 
 namespace {
 
-constexpr int kSelThreads = 256;
-constexpr int kSelTile = 2048;  // probes per tile: 8 per thread, 32 ballot words
+// A tile's probes are taken two a thread: the passes are as long as a thread's
+// chain of loads (8 probes a thread: flags 8.8 us, scan 4.1, scatter 5.3 for
+// 36,864 probes; 2 a thread: flags 5.6 us, scan and scatter in one 3.5).
+constexpr int kSelThreads = 1024;
+constexpr int kSelTile = 2048;  // probes per tile: 32 ballot words
 
 __device__ __forceinline__ int neighbour_sum(const int16_t* blocks, int wx, int wy, int wz, int x, int y, int z) {
     int s = 0;
@@ -106,17 +110,10 @@ __device__ __forceinline__ int group_scan(int v, int* s_wave, int* total) {
     return x + before;
 }
 
-__global__ __launch_bounds__(1024) void select_scan_kernel(SelectArgs a) {
+// The special requests, after `running` probes selected by the grid, and the
+// count (one workgroup).
+__device__ __forceinline__ void select_special(const SelectArgs& a, int running) {
     __shared__ int s_wave[16];
-    int running = 0;
-    for (int base = 0; base < a.n_tiles; base += blockDim.x) {
-        const int i = base + threadIdx.x;
-        const int v = i < a.n_tiles ? a.tile_counts[i] : 0;
-        int total;
-        const int incl = group_scan(v, s_wave, &total);
-        if (i < a.n_tiles) a.tile_counts[i] = running + incl - v;  // now the tile's offset
-        running += total;
-    }
     for (int base = 0; base < a.n_special; base += blockDim.x) {
         const int i = base + threadIdx.x;
         int4 q = make_int4(0, 0, 0, 0);
@@ -137,18 +134,39 @@ __global__ __launch_bounds__(1024) void select_scan_kernel(SelectArgs a) {
     if (threadIdx.x == 0) a.count[0] = min(running, a.n);
 }
 
+__global__ __launch_bounds__(1024) void select_scan_kernel(SelectArgs a) {
+    __shared__ int s_wave[16];
+    int running = 0;
+    for (int base = 0; base < a.n_tiles; base += blockDim.x) {
+        const int i = base + threadIdx.x;
+        const int v = i < a.n_tiles ? a.tile_counts[i] : 0;
+        int total;
+        const int incl = group_scan(v, s_wave, &total);
+        if (i < a.n_tiles) a.tile_counts[i] = running + incl - v;  // now the tile's offset
+        running += total;
+    }
+    select_special(a, running);
+}
+
+// SUM: tile_counts holds counts, and one workgroup more than tiles takes the
+// special requests; else it holds offsets, from select_scan_kernel.
+template <bool SUM>
 __global__ __launch_bounds__(kSelThreads) void select_scatter_kernel(SelectArgs a) {
     constexpr int kWords = kSelTile / 64;
     __shared__ int s_pref[kWords];
     const int tile = blockIdx.x;
-    const unsigned long long* words = a.bits + (size_t)tile * kWords;
-    if (threadIdx.x < kWords) {
-        int s = 0;
-        for (int c = 0; c < (int)threadIdx.x; ++c) s += __popcll(words[c]);
-        s_pref[threadIdx.x] = s;
+    int offset = 0;
+    if constexpr (SUM) {
+        offset = sum_before(a.tile_counts, tile);
+        if (tile == a.n_tiles) {
+            select_special(a, offset);
+            return;
+        }
     }
+    const unsigned long long* words = a.bits + (size_t)tile * kWords;
+    if (threadIdx.x < 64) word_prefix(words, kWords, s_pref);
     __syncthreads();
-    const int offset = a.tile_counts[tile];
+    if constexpr (!SUM) offset = a.tile_counts[tile];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int k = 0; k < kSelTile / kSelThreads; ++k) {
         const int c = k * (kSelThreads / 64) + wave;
@@ -191,9 +209,12 @@ size_t select_bits_bytes(int n_probes) { return select_tiles(n_probes) * (kSelTi
 hipError_t launch_select(const SelectArgs& a, hipStream_t stream) {
     if (a.n_tiles > 0)
         hipLaunchKernelGGL(select_flags_kernel, dim3(a.n_tiles), dim3(kSelThreads), 0, stream, a);
-    hipLaunchKernelGGL(select_scan_kernel, dim3(1), dim3(1024), 0, stream, a);
-    if (a.n_tiles > 0)
-        hipLaunchKernelGGL(select_scatter_kernel, dim3(a.n_tiles), dim3(kSelThreads), 0, stream, a);
+    if (a.n_tiles <= kSumTiles) {
+        hipLaunchKernelGGL(select_scatter_kernel<true>, dim3(a.n_tiles + 1), dim3(kSelThreads), 0, stream, a);
+    } else {
+        hipLaunchKernelGGL(select_scan_kernel, dim3(1), dim3(1024), 0, stream, a);
+        hipLaunchKernelGGL(select_scatter_kernel<false>, dim3(a.n_tiles), dim3(kSelThreads), 0, stream, a);
+    }
     return hipGetLastError();
 }
 
