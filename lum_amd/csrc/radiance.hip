@@ -335,8 +335,8 @@ __device__ __forceinline__ void radiance_lane_body(const RadianceArgs& a, const 
 // The march is bound by vector issue and by the latency of its gathers, so
 // waves in flight count: 80 scalar registers and 64 vector registers keep
 // eight waves on a SIMD (at 96 scalar registers seven fit, 6% slower).
-// 128 x 128 x 32 blocks, 128 rays, FP16 field: 5065 us with one body for every
-// ray, 4205 us now; 24 worlds in a batch 2610 -> 2324 us.
+// 256 x 256 x 32 blocks, 128 rays, FP16 field: 5057 us with one body for every
+// ray, 3981 us now; 24 worlds in a batch, glossy queries included: 2613 -> 2184.
 
 // Wave-uniform loads through the scalar cache: data that no thread of this
 // launch writes, at an address that is the same for the whole wave.
