@@ -1485,8 +1485,7 @@ static_assert(sizeof(GridBatch) <= 4096, "kernel arguments are limited to 4 KiB"
 
 __global__ void __launch_bounds__(256) march_grid_batch_kernel(GridBatch b) {
     __shared__ GridLds lds;
-    int i = 0;
-    while (i + 1 < b.n && b.begin[i + 1] <= (int)blockIdx.x) ++i;
+    const int i = last_begin(b.begin, b.n, (int)blockIdx.x);
     march_grid_tile(b.g[i], (int)blockIdx.x - b.begin[i], lds);
 }
 
