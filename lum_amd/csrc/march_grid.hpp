@@ -74,7 +74,8 @@ __device__ __forceinline__ RayHit refine_grid(const Args& a, const MarchRay& m, 
 // it stays in plain air, so two samples are taken at a time: the second's grid
 // byte is on its way before the first's arrives, and counts only if the first
 // was air.  (A second sample after a first outside the world may lie further
-// out: its index is clamped.)  Grid indices are formed in floats, exact below
+// out: indices are clamped, so that not even a grid that is being rewritten by
+// an unordered map leads a read out of it.)  Grid indices are formed in floats, exact below
 // 2^24: six 2-cycle operations and a conversion instead of three conversions
 // and two 4-cycle multiply-adds.
 //
@@ -132,7 +133,7 @@ __device__ __forceinline__ RayHit cast_ray_grid(const Args& a, f3 o, f3 d) {
         int taken = 0;
         do {
             s0 = sample(fraction);
-            b0 = gld(a.grid, (unsigned)s0.index);
+            b0 = gld(a.grid, (unsigned)fminf(s0.index, last));
             s1 = sample(s0.next);
             b1 = gld(a.grid, (unsigned)fminf(s1.index, last));
             second = b0 == 0 && s0.next < a.max_dist && left > taken + 1;
