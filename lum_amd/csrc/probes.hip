@@ -10,15 +10,18 @@
 //   select_flags_kernel   one workgroup per tile of 2048 probes: the flags as
 //                         64-bit wave ballots (one word per 64 probes) and
 //                         the tile's count;
-//   select_scan_kernel    one workgroup: exclusive scan of the tile counts,
-//                         then the specials in order (kept = inside the world
-//                         and its probe not flagged; repeats are kept, as the
-//                         reference marks only grid probes as taken), written
-//                         after the grid probes up to one entry per probe
-//                         (the capacity of the reference's request buffer),
-//                         count stored;
 //   select_scatter_kernel one workgroup per tile: each flagged probe goes to
-//                         tile offset + rank within the tile.
+//                         tile offset + rank within the tile, the offset
+//                         being the sum of the counts before; one workgroup
+//                         more takes the specials in order (kept = inside the
+//                         world and its probe not flagged; repeats are kept,
+//                         as the reference marks only grid probes as taken),
+//                         written after the grid probes up to one entry per
+//                         probe (the capacity of the reference's request
+//                         buffer), and stores the count;
+//   select_scan_kernel    (more than kSumTiles tiles) one workgroup, between
+//                         the two: exclusive scan of the tile counts, then the
+//                         specials and the count.
 //
 // Field shift restates shift_radiance (src/renderer/src/internal_render.cpp:
 // 1218-1335): the intersection of the field and the field moved by `shift`
