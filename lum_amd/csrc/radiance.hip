@@ -723,9 +723,9 @@ static hipError_t launch_store(const RadianceArgs& a, hipStream_t stream) {
             hipLaunchKernelGGL((radiance_chunk_kernel<STORE, true>), dim3(grid), dim3(bs), lds, stream, a);
         else
             hipLaunchKernelGGL((radiance_chunk_kernel<STORE, false>), dim3(grid), dim3(bs), lds, stream, a);
-        return hipGetLastError();
+    } else {
+        hipLaunchKernelGGL((radiance_kernel<STORE, TRACED, OCC, K>), dim3(grid), dim3(bs), lds, stream, a);
     }
-    hipLaunchKernelGGL((radiance_kernel<STORE, TRACED, OCC, K>), dim3(grid), dim3(bs), lds, stream, a);
     return hipGetLastError();
 }
 
