@@ -329,7 +329,7 @@ int launcher_map(Launcher* L, lumx_world* const* worlds, int n, const int* n_mod
         launch_begin_off[k] = off;
         off += round_up(((size_t)launch_count[k] + 1) * sizeof(int), 256);
     }
-    long long groups = 0, slots = 0;
+    long long groups = 0, slots = 0, bits = 0;
     for (int i = 0; i < m; ++i) {
         lumx_world* w = worlds[i];
         MapWorldDesc& d = desc[i];
@@ -363,6 +363,8 @@ int launcher_map(Launcher* L, lumx_world* const* worlds, int n, const int* n_mod
         groups += (map_commit_elements(d) + 255) / 256;
         d.slot_begin = (int)slots;
         slots += d.hi - st;
+        d.bits_begin = (int)bits;
+        bits += named_slots(w) - st;
     }
     if (groups > (1ll << 31) - 1) return fail(LUMX_EINVAL, "batched map too large");
     const size_t need = off;
@@ -426,7 +428,7 @@ int launcher_map(Launcher* L, lumx_world* const* worlds, int n, const int* n_mod
     for (size_t k = 0; k < n_launches; ++k)
         HIP_TRY(launch_map_batch((const MapArgs*)(dv + launch_off[k]), (const int*)(dv + launch_begin_off[k]),
                                  launch_count[k], total_groups[k], s));
-    HIP_TRY(launch_palette_bits_batch(d_dev, m, (int)slots, s));
+    HIP_TRY(launch_palette_bits_batch(d_dev, m, (int)bits, s));
     HIP_TRY(launch_march_grid_batch(grids.data(), m, s));
     for (int i = 0; i < m; ++i) {
         worlds[i]->prev_counter = worlds[i]->counter;

@@ -219,12 +219,27 @@ WorldView lumx::view_of(const lumx_world* w) {
     return v;
 }
 
+int lumx::named_slots(const lumx_world* w) {
+    return std::max(w->host_stale ? w->dev_counter_bound : std::max(w->counter, w->prev_counter), w->origin_slots);
+}
+
+int lumx::kept_slots(const lumx_world* w) { return std::max(named_slots(w), w->origin_top); }
+
+void lumx::scan_origin(lumx_world* w) {
+    if (!w->origin_ids_dirty) return;
+    int top = w->desc.static_blocks;
+    for (int16_t b : w->origin) top = std::max(top, b + 1);
+    w->origin_slots = top;
+    w->origin_top = std::max(w->origin_top, top);
+    w->origin_ids_dirty = false;
+}
+
 GridArgs lumx::grid_args(const lumx_world* w) {
     GridArgs g;
     g.empty_bits = w->empty_bits;
     g.blocks = w->blocks;
     g.slot_mask = w->slot_mask;
-    g.slots = w->desc.palette_slots;
+    g.slots = named_slots(w);
     g.grid = w->grid;
     g.escape = w->escape;
     g.wx = w->desc.size[0];
@@ -492,7 +507,7 @@ int lumx::world_snapshot_async(lumx_world* w, hipStream_t s, bool field_only) {
     if (rc) return rc;
     if (w->stage_pending) HIP_TRY(hipEventSynchronize(w->stage_done));
     w->stage_pending = false;
-    const int used = std::max(w->counter, w->prev_counter);
+    const int used = kept_slots(w);
     if (field_only && !(w->snap_static_valid && used == w->snap_used))
         return fail(LUMX_EINVAL, "no snapshot of the world's static state to keep");
     rc = world_snapshot_reserve(w, used, s);
@@ -512,7 +527,7 @@ int lumx::world_snapshot_async(lumx_world* w, hipStream_t s, bool field_only) {
 }
 
 int lumx::world_snapshot_static(lumx_world* w) {
-    const int used = std::max(w->counter, w->prev_counter);
+    const int used = kept_slots(w);
     int rc = world_snapshot_reserve(w, used, nullptr);
     if (rc) return rc;
     HIP_TRY(hipMemcpy(w->snap_host, w->dev_mem, snap_static_bytes(w, used), hipMemcpyDeviceToHost));
@@ -609,6 +624,7 @@ int lumx_world_create(lumx_context_t c, const lumx_world_desc* d, lumx_world_t* 
     w->static_palette.assign((size_t)d->static_blocks * 4096, 0);
     w->counter = d->static_blocks;
     w->prev_counter = d->static_blocks;
+    w->origin_slots = w->origin_top = d->static_blocks;
     w->tune = default_tuning();
     w->device_bytes = lumx::world_bytes(w);
     hipError_t e = world_alloc_device(w);
@@ -882,10 +898,11 @@ static int sync_host_state(lumx_world* w) {
     return LUMX_OK;
 }
 
-// Occupancy bits of the dynamic slots after the palette changed on device.
+// Occupancy bits of the dynamic slots after the palette changed on device
+// (models write into the slots of the map and into those of the origin world).
 static int commit_palette_bits(lumx_world* w, hipStream_t s) {
     const int st = w->desc.static_blocks;
-    const int hi = std::max(w->counter, w->prev_counter);
+    const int hi = named_slots(w);
     if (hi > st) HIP_TRY(launch_palette_bits(w->palette, st, hi - st, w->pal_bits, w->slot_mask, 0, s));
     HIP_TRY(launch_march_grid(grid_args(w), s));
     w->prev_counter = w->counter;
@@ -900,6 +917,7 @@ int lumx_world_upload_blocks(lumx_world_t w, void* stream) {
     if (rc0) return rc0;
     w->current = w->origin;
     w->counter = w->desc.static_blocks;
+    scan_origin(w);
     hipStream_t s = pick_stream(w->ctx, stream);
     int rc = commit_blocks(w, s);
     if (rc) return rc;
@@ -1084,16 +1102,8 @@ static int plan_map_launches(lumx_world* w, int n, const lumx_model_t* models, c
     SmallBuf<MapArgs, kNoAllocModels> args(std::max(n, 1));
     SmallBuf<int, kNoAllocModels> layer(std::max(n, 1), 0);
     SmallBuf<char, kNoAllocModels> negative(std::max(n, 1), 0);
-    if (w->origin_ids_dirty) {
-        w->origin_has_dynamic = false;
-        for (int16_t b : w->origin)
-            if (b >= st) {
-                w->origin_has_dynamic = true;
-                break;
-            }
-        w->origin_ids_dirty = false;
-    }
-    const bool aliasing = w->origin_has_dynamic;
+    scan_origin(w);
+    const bool aliasing = w->origin_slots > st;
     for (int i = 0; i < n; ++i) {
         const lumx_placement& p = pl[i];
         MapArgs& a = args[i];
@@ -1340,8 +1350,11 @@ static int map_device(lumx_world_t w, int n, const lumx_model_t* models, const l
     if (rc) return rc;
     // The claims took the place of every slot's mask.
     const int from = w->slot_mask ? 0 : st, fill = w->slot_mask ? slots : 0;
-    HIP_TRY(launch_palette_bits(w->palette, from, bound - from, w->pal_bits, w->slot_mask, fill, s));
-    HIP_TRY(launch_march_grid(grid_args(w), s));
+    const int named = std::max(bound, w->origin_slots);
+    HIP_TRY(launch_palette_bits(w->palette, from, named - from, w->pal_bits, w->slot_mask, fill, s));
+    GridArgs ga = grid_args(w);
+    ga.slots = named;
+    HIP_TRY(launch_march_grid(ga, s));
     w->host_stale = true;
     w->dev_counter_bound = (int)std::min<long long>(slots, st + total);
     if (capturing) return LUMX_OK;
@@ -1588,7 +1601,7 @@ static int radiance_launch(lumx_world* w, const int32_t* req, int n_req, const l
         t.eb_lds = 1;
         base += 4 * (size_t)a.eb_words;
     }
-    const int used_slots = w->host_stale ? w->dev_counter_bound : std::max(w->counter, w->prev_counter);
+    const int used_slots = named_slots(w);
     if (tune.lds_palette_bits && base + 4 * (size_t)used_slots * 128 <= kLdsBudget) {
         t.pb_lds = 1;
         a.pb_words = used_slots * 128;

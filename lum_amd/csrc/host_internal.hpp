@@ -117,8 +117,11 @@ struct lumx_world {
     // Device blockify.
     int16_t* origin_dev = nullptr;          // device copy of the origin world
     bool origin_dirty = true;               // origin changed since its last upload
-    bool origin_ids_dirty = true;           // origin changed since origin_has_dynamic was computed
-    bool origin_has_dynamic = false;        // an origin id >= static_blocks (a slot two blocks may share)
+    bool origin_ids_dirty = true;           // origin changed since origin_slots was computed
+    int origin_slots = 0;                   // 1 + the highest id of the origin world, at least static_blocks:
+                                            // above it an origin world names dynamic slots itself
+                                            // (two blocks may share one, and models write into them)
+    int origin_top = 0;                     // the highest origin_slots so far
     int* blockify_state = nullptr;          // device: counter, copy bound, overflow
     void* blockify_scratch = nullptr;       // device: model boxes, ballot words, tile counts
     size_t blockify_scratch_bytes = 0;
@@ -203,6 +206,14 @@ void compact_args(const lumx_world* w, RadianceArgs* a);
 void glossy_args(lumx_world* w, const uint8_t* matnorm, const float* depth, int width, int height,
                  const lumx_camera* cam, float max_dist, int max_steps, float* out, int32_t* keys, GlossyArgs* a);
 WorldView view_of(const lumx_world* w);
+// Slots that w's blocks may name: those of the last two maps (after a device
+// map a bound) and those that the origin world names.
+int named_slots(const lumx_world* w);
+// Slots that may hold voxels: those, and the ones earlier origin worlds named
+// (nothing clears them).
+int kept_slots(const lumx_world* w);
+// origin_slots and origin_top of the present origin world.
+void scan_origin(lumx_world* w);
 // The march grid of w's blocks, built from its empty-block bits.
 GridArgs grid_args(const lumx_world* w);
 bool stream_capturing(hipStream_t s);

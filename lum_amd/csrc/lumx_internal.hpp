@@ -78,7 +78,8 @@ struct GridArgs {
     const uint8_t* slot_mask;  // per slot (nullptr: unknown): which of its 8^3 octants hold a voxel
     uint8_t* grid;
     uint8_t* escape;
-    int wx, wy, wz, n_blocks, slots;
+    int wx, wy, wz, n_blocks;
+    int slots;              // slots whose octants are known: a block with an id above may hold voxels in all
     int tiles;              // march_grid_tiles(wx, wy, wz)
 };
 #if defined(__HIPCC__)
@@ -322,8 +323,9 @@ struct MapWorldDesc {
     unsigned long long stage_slots;   // byte offset of the staged slot blocks (slots st .. counter - 1)
     int group_begin;          // first workgroup of this world in the commit launch
     int n_blocks;
-    int st, hi;               // slots st .. hi - 1 are copied and get their occupancy bits
+    int st, hi;               // slots st .. hi - 1 are copied
     int counter;
+    int bits_begin;           // first slot of this world in the concatenated ranges that get occupancy bits (from st)
     int slot_begin;           // first slot of this world in the concatenated st .. hi - 1 ranges
 };
 // origin blocks + their empty-block bits + copy list + counter of every

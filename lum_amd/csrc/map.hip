@@ -208,8 +208,8 @@ __global__ void __launch_bounds__(256) map_copies_batch_kernel(const MapWorldDes
 // One workgroup of 128 threads per slot: the slot's voxel-occupancy words.
 __global__ void __launch_bounds__(128) palette_bits_batch_kernel(const MapWorldDesc* d, int n) {
     const int b = (int)blockIdx.x;
-    const MapWorldDesc& w = d[world_of<&MapWorldDesc::slot_begin>(d, n, b)];
-    const int slot = w.st + (b - w.slot_begin);
+    const MapWorldDesc& w = d[world_of<&MapWorldDesc::bits_begin>(d, n, b)];
+    const int slot = w.st + (b - w.bits_begin);
     const uint8_t* src = w.palette + ((size_t)slot << 12) + threadIdx.x * 32;
     const uint4 a0 = ((const uint4*)src)[0];
     const uint4 a1 = ((const uint4*)src)[1];

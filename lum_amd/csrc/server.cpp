@@ -751,7 +751,7 @@ int lumx_server_add_world(lumx_server_t s, lumx_world_t w, int* id) {
         // block), else to the host, into its pinned snapshot.
         HIP_TRY(hipDeviceSynchronize());  // work on the world may be queued on any stream
         // Its pinned snapshot now, so no eviction allocates while serving.
-        int rc = world_snapshot_reserve(w, std::max(w->counter, w->prev_counter), s->copy_stream);
+        int rc = world_snapshot_reserve(w, kept_slots(w), s->copy_stream);
         if (rc) return rc;
         size_t off = 0;
         if (s->arena.take(w->device_bytes, &off)) {
