@@ -1084,6 +1084,17 @@ static int blockify(lumx_world* w, const lumx_placement& p) {
     return LUMX_OK;
 }
 
+// Voxels and workgroup tiles of a placed model's dispatch box.
+static void set_dispatch(MapArgs& a, const lumx_placement& p) {
+    a.nx = p.groups[0] * 4; a.ny = p.groups[1] * 4; a.nz = p.groups[2] * 4;
+    a.tiles_x = (a.nx + 15) / 16;
+    a.tiles_y = a.ny / 4;
+}
+
+static int check_dispatch(const MapArgs& a, int i) {
+    return map_tiles(a) >= (1ll << 28) ? fail(LUMX_EINVAL, "model %d dispatch too large", i) : LUMX_OK;
+}
+
 // map.comp for each placed model, in order, over the current device world.
 // Models go in layers: a model's layer is one more than that of the last
 // earlier model whose write box (the voxels its dispatch covers) intersects
@@ -1114,15 +1125,12 @@ static int plan_map_launches(lumx_world* w, int n, const lumx_model_t* models, c
         a.palette_slots = w->desc.palette_slots;
         a.static_count = st;
         a.mx = models[i]->size[0]; a.my = models[i]->size[1]; a.mz = models[i]->size[2];
-        a.nx = p.groups[0] * 4; a.ny = p.groups[1] * 4; a.nz = p.groups[2] * 4;
+        set_dispatch(a, p);
         a.shift_x = p.shift[0]; a.shift_y = p.shift[1]; a.shift_z = p.shift[2];
         for (int r = 0; r < 3; ++r)
             for (int c = 0; c < 4; ++c) a.m[r * 4 + c] = p.minv[c * 4 + r];
         a.cls = 7;
-        a.tiles_x = (a.nx + 15) / 16;
-        a.tiles_y = a.ny / 4;
-        if (map_tiles(a) >= (1ll << 28))
-            return fail(LUMX_EINVAL, "model %d dispatch too large", i);
+        if (int rc = check_dispatch(a, i)) return rc;
         a.div_tiles_x = make_divisor((uint32_t)std::max(a.tiles_x, 1));
         a.div_tiles_y = make_divisor((uint32_t)std::max(a.tiles_y, 1));
         negative[i] = a.shift_x < 0 || a.shift_y < 0 || a.shift_z < 0;
@@ -1171,9 +1179,10 @@ static int plan_map_launches(lumx_world* w, int n, const lumx_model_t* models, c
 }  // extern "C++"
 
 // The launches of plan_map_launches in order, up to kMapGroup models per
-// launch (descriptors as the kernel argument).  Allocates nothing.
+// launch (descriptors as the kernel argument).  Allocates nothing.  Without
+// `launch` only the checks.
 static int launch_models(lumx_world* w, int n, const lumx_model_t* models, const lumx_placement* pl,
-                         hipStream_t s) {
+                         hipStream_t s, bool launch = true) {
     return plan_map_launches(w, n, models, pl, [&](const MapArgs* group, int count) -> int {
         MapGroup g;
         g.n = 0;
@@ -1189,13 +1198,27 @@ static int launch_models(lumx_world* w, int n, const lumx_model_t* models, const
                 g.n++;
             }
             if (g.n == kMapGroup || (k == count && g.n > 0)) {
-                HIP_TRY(launch_map_group(g, s));
+                if (launch) HIP_TRY(launch_map_group(g, s));
                 g.n = 0;
                 g.begin[0] = 0;
             }
         }
         return LUMX_OK;
     });
+}
+
+// Every check of launch_models, before a map changes the world: a map that is
+// refused half way would leave blocks without their march grid.
+static int check_models(lumx_world* w, int n, const lumx_model_t* models, const lumx_placement* pl) {
+    long long total = 0;
+    for (int i = 0; i < n; ++i) {
+        MapArgs a;
+        set_dispatch(a, pl[i]);
+        if (int rc = check_dispatch(a, i)) return rc;
+        total += std::max(map_tiles(a), 0ll);
+    }
+    if (total <= (1ll << 31) - 1) return LUMX_OK;  // no launch can be too large
+    return launch_models(w, n, models, pl, nullptr, false);
 }
 
 // Block box of blockify_mesh for a placed model (internal_render.cpp:1032-1037).
@@ -1219,6 +1242,7 @@ static int map_device(lumx_world_t w, int n, const lumx_model_t* models, const l
     for (int i = 0; i < n; ++i)
         if (!models[i] || models[i]->ctx != w->ctx) return fail(LUMX_EINVAL, "model %d invalid", i);
     REQUIRE_RESIDENT(w);
+    if (int rc = check_models(w, n, models, pl)) return rc;
     HIP_TRY(hipSetDevice(w->ctx->device));
     hipStream_t s = pick_stream(w->ctx, stream);
     const bool capturing = stream_capturing(s);
@@ -1345,16 +1369,24 @@ static int map_device(lumx_world_t w, int n, const lumx_model_t* models, const l
     // previous map's counters.
     const int prev_bound = w->host_stale ? w->dev_counter_bound : std::max(w->counter, w->prev_counter);
     const int bound = (int)std::min<long long>(slots, std::max<long long>(st + total, prev_bound));
-    HIP_TRY(launch_blockify(a, bound - st, s));
-    int rc = launch_models(w, n, models, pl, s);
-    if (rc) return rc;
-    // The claims took the place of every slot's mask.
-    const int from = w->slot_mask ? 0 : st, fill = w->slot_mask ? slots : 0;
-    const int named = std::max(bound, w->origin_slots);
-    HIP_TRY(launch_palette_bits(w->palette, from, named - from, w->pal_bits, w->slot_mask, fill, s));
-    GridArgs ga = grid_args(w);
-    ga.slots = named;
-    HIP_TRY(launch_march_grid(ga, s));
+    // Until the last of these launches the claims stand where the march grid does.
+    const int rc = [&]() -> int {
+        HIP_TRY(launch_blockify(a, bound - st, s));
+        if (int e = launch_models(w, n, models, pl, s)) return e;
+        // The claims took the place of every slot's mask.
+        const int from = w->slot_mask ? 0 : st, fill = w->slot_mask ? slots : 0;
+        const int named = std::max(bound, w->origin_slots);
+        HIP_TRY(launch_palette_bits(w->palette, from, named - from, w->pal_bits, w->slot_mask, fill, s));
+        GridArgs ga = grid_args(w);
+        ga.slots = named;
+        HIP_TRY(launch_march_grid(ga, s));
+        return LUMX_OK;
+    }();
+    if (rc) {
+        // A device error: marches read the blocks from now on (recorded launches have not run).
+        if (!capturing) w->grid = w->escape = nullptr;
+        return rc;
+    }
     w->host_stale = true;
     w->dev_counter_bound = (int)std::min<long long>(slots, st + total);
     if (capturing) return LUMX_OK;
@@ -1417,6 +1449,8 @@ int lumx::map_plan(lumx_world* w, int n, const lumx_model_t* models, const lumx_
 int lumx_map_models_placed(lumx_world_t w, int n, const lumx_model_t* models, const lumx_placement* pl,
                            void* stream) {
     int rc0 = map_check(w, n, models, pl);
+    if (rc0) return rc0;
+    rc0 = check_models(w, n, models, pl);
     if (rc0) return rc0;
     rc0 = map_prepare(w, n, pl);
     if (rc0) return rc0;
