@@ -236,7 +236,8 @@ int lumx_world_palette_counter(lumx_world_t w, int* out);
  * NULL for every probe in x-fastest order (n_requests ignored).  Reads the
  * current field, writes a new one (Jacobi), then makes it current.  A list
  * dispatches n_requests / size probes, at most the world's block count (the
- * capacity of the reference's request buffer; more is LUMX_EINVAL).  Entries
+ * capacity of the reference's request buffer; more is LUMX_EINVAL; so are
+ * more than 2^32 threads, one a ray or two or four rays, in one launch).  Entries
  * outside the world are skipped; where several dispatched entries name one
  * probe, the last of them is the one stored. */
 int lumx_radiance_update(lumx_world_t w, const int32_t* requests_dev, int n_requests,

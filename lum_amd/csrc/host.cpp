@@ -1598,6 +1598,15 @@ static int radiance_launch(lumx_world* w, const int32_t* req, int n_req, const l
     // check that can fail); the scatter that applies it consumes (and resets)
     // the claims.
     if (a.staged && apply) a.claim = w->upd_claim;
+    // Threads of the launch (the persistent kernel of variant 1 takes any number of rays).
+    if (tune.variant != 1) {
+        const int K = tune.variant == 2 || traced ? 1 : rays_per_lane_for(p->rays, tune.rays_per_lane);
+        const long long lanes = tune.variant == 3 && !traced ? 64ll * a.n_probes / tune.probes_per_batch
+                                                              : (long long)a.n_probes * (p->rays / K);
+        if (lanes > 0xffffffffll - 1024)
+            return fail(LUMX_EINVAL, "%d probes of %d rays are more than one launch takes (2^32 threads): update "
+                                     "them in parts (size, shift)", a.n_probes, p->rays);
+    }
     if (tune.variant == 3 && !traced) {
         if (p->rays != 64) return fail(LUMX_EINVAL, "the refill variant takes 64 rays per probe");
         HIP_TRY(launch_claim(a, s));

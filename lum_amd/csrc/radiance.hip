@@ -225,8 +225,8 @@ __device__ __forceinline__ void store_probe(const RadianceArgs& a, int wg, int p
 }
 
 // K rays per lane.  tid is the thread's index within this world's launch
-// range, which starts on a workgroup boundary; a probe owns L = R / K
-// consecutive threads.
+// range (unsigned: a single world's launch may hold 2^32 - 1 threads), which
+// starts on a workgroup boundary; a probe owns L = R / K consecutive threads.
 //
 // The probe total is reduced in one fixed order for every K: per chunk of
 // C = min(R, 64) rays a butterfly (v[i] += v[i ^ s], s = C/2 .. 1), then the
@@ -239,14 +239,14 @@ __device__ __forceinline__ void store_probe(const RadianceArgs& a, int wg, int p
 //   or o = 0, 2, 1, 3 (Kw = 4): stage C/2 pairs rays p and p + C/2 (o = 0, 2
 //   for Kw = 4), stage C/4 pairs their sums.
 template <int STORE, bool TRACED, bool OCC, int K>
-__device__ __forceinline__ void radiance_lane_body(const RadianceArgs& a, const int time_seed, const int tid, f3* chunk_sum) {
+__device__ __forceinline__ void radiance_lane_body(const RadianceArgs& a, const int time_seed, const uint32_t tid, f3* chunk_sum) {
     const int R = a.rays;
     constexpr int LOG2K = K == 1 ? 0 : (K == 2 ? 1 : 2);
     const int L = R >> LOG2K;  // K > 1: R is a power of two
-    int wg = K == 1 ? (a.log2_rays >= 0 ? (tid >> a.log2_rays) : tid / R) : (tid >> (a.log2_rays - LOG2K));
+    int wg = (int)(K == 1 ? (a.log2_rays >= 0 ? (tid >> a.log2_rays) : tid / (uint32_t)R) : (tid >> (a.log2_rays - LOG2K)));
     // With L >= 64 a wave holds lanes of one probe: keep the probe on the scalar unit.
     if (L >= 64) wg = __builtin_amdgcn_readfirstlane(wg);
-    const int m = tid - wg * L;
+    const int m = (int)(tid - (uint32_t)wg * (uint32_t)L);
     int px = 0, py = 0, pz = 0, key = wg;
     const bool valid = probe_coords(a, wg, &px, &py, &pz, &key);
     const f3 zero = {0.0f, 0.0f, 0.0f};
@@ -430,18 +430,18 @@ __device__ __forceinline__ unsigned escape_octant(f3 d) {
 // UNI: R >= 64, a wave's rays belong to one probe.  tid as for
 // radiance_lane_body.
 template <int STORE, bool UNI>
-__device__ __forceinline__ void radiance_chunk_body(const RadianceArgs& a, const int time_seed, const int tid, f3* chunk_sum) {
+__device__ __forceinline__ void radiance_chunk_body(const RadianceArgs& a, const int time_seed, const uint32_t tid, f3* chunk_sum) {
     const WorldView& w = a.world;
     const int R = a.rays, lane = threadIdx.x & 63;
     int wg, k = 0, r;  // probe, chunk of the probe, ray of the probe
     if constexpr (UNI) {
-        const int c = __builtin_amdgcn_readfirstlane(tid >> 6), per = R >> 6;
+        const int c = __builtin_amdgcn_readfirstlane((int)(tid >> 6)), per = R >> 6;
         wg = a.log2_rays >= 0 ? c >> (a.log2_rays - 6) : c / per;
         k = c - wg * per;
         r = k * 64 + lane;
     } else {
-        wg = tid >> a.log2_rays;
-        r = tid & (R - 1);
+        wg = (int)(tid >> a.log2_rays);
+        r = (int)tid & (R - 1);
     }
     int x = 0, y = 0, z = 0, key = wg;
     const bool valid = probe_coords(a, wg, &x, &y, &z, &key);
@@ -522,7 +522,7 @@ __device__ __forceinline__ void radiance_chunk_body(const RadianceArgs& a, const
 template <int STORE, bool UNI>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8))) radiance_chunk_kernel(RadianceArgs a) {
     extern __shared__ f3 chunk_sum[];
-    radiance_chunk_body<STORE, UNI>(a, a.time_seed, (int)(blockIdx.x * blockDim.x + threadIdx.x), chunk_sum);
+    radiance_chunk_body<STORE, UNI>(a, a.time_seed, blockIdx.x * blockDim.x + threadIdx.x, chunk_sum);
 }
 
 template <int STORE, bool TRACED, bool OCC, int K>
@@ -668,7 +668,7 @@ radiance_batch_kernel(const RadianceArgs* args, const int* begin, int n_worlds, 
     // six waves a SIMD: 2672 us for 24 worlds, 2389 us without it.
     const RadianceArgs& a = *constant_args(args + lo);
     const int time_seed = a.time_seed + (frame ? *frame : 0);
-    const int tid = (int)(blockIdx.x * blockDim.x + threadIdx.x) - begin[lo];
+    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x - (uint32_t)begin[lo];
     if constexpr (K == 1 && !OCC) {
         if (a.rays >= 64) radiance_chunk_body<STORE, true>(a, time_seed, tid, chunk_sum);
         else radiance_chunk_body<STORE, false>(a, time_seed, tid, chunk_sum);
