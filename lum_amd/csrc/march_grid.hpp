@@ -13,7 +13,7 @@ namespace lumx {
 // Voxels of one block in a row cost one load each: the block id is fetched
 // only when the block changes.
 template <class Args>
-__device__ __forceinline__ RayHit refine_grid(const Args& a, const MarchRay& m, f3 bh, int key, int id) {
+LUMX_HD RayHit refine_grid(const Args& a, const MarchRay& m, f3 bh, int key, int id) {
     const WorldView& w = a.world;
     const int kx = w.wx + 2, kxy = kx * (w.wy + 2);
     const f3 d = m.d, inv = m.inv;
@@ -23,7 +23,7 @@ __device__ __forceinline__ RayHit refine_grid(const Args& a, const MarchRay& m, 
         const int ix = (int)v.x, iy = (int)v.y, iz = (int)v.z;
         // Block 0 also holds -15 .. -1 (the shader's truncating division).
         const int bx = block_axis(ix), by = block_axis(iy), bz = block_axis(iz);
-        const int k = bx + __mul24(by, kx) + __mul24(bz, kxy);
+        const int k = bx + (int)(mul24((unsigned)by, (unsigned)kx) + mul24((unsigned)bz, (unsigned)kxy));
         if (k != key) {
             key = k;
             id = 0;
@@ -65,6 +65,15 @@ __device__ __forceinline__ RayHit refine_grid(const Args& a, const MarchRay& m, 
     return r;
 }
 
+// A float index into the grid, within it whatever its value (v_med3_f32).
+LUMX_HD unsigned clamp_index(float index, float last) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (unsigned)__builtin_amdgcn_fmed3f(index, 0.0f, last);
+#else
+    return (unsigned)fminf(fmaxf(index, 0.0f), last);
+#endif
+}
+
 // cast_ray over the world's march grid (a.grid, which takes slot 0 as air).
 // The ray's first sample lies in the world or in the block around it, and no
 // axis of d is longer than 16: then no sample lies further out, the next one
@@ -74,10 +83,10 @@ __device__ __forceinline__ RayHit refine_grid(const Args& a, const MarchRay& m, 
 // it stays in plain air, so two samples are taken at a time: the second's grid
 // byte is on its way before the first's arrives, and counts only if the first
 // was air.  (A second sample after a first outside the world may lie further
-// out: indices are clamped, so that not even a grid that is being rewritten by
-// an unordered map leads a read out of it.)  Grid indices are formed in floats, exact below
-// 2^24: six 2-cycle operations and a conversion instead of three conversions
-// and two 4-cycle multiply-adds.
+// out: indices are clamped at both ends, so that not even a grid that is being
+// rewritten by an unordered map leads a read out of it.)  Grid indices are
+// formed in floats, exact below 2^24: six 2-cycle operations and a conversion
+// instead of three conversions and two 4-cycle multiply-adds.
 //
 // In a block that holds something, samples lie half a voxel apart.  The grid
 // byte tells its empty octants: n samples in one are passed by at once.
@@ -92,7 +101,7 @@ __device__ __forceinline__ RayHit refine_grid(const Args& a, const MarchRay& m, 
 // 1 takes 320 us for a world with 32 models (48 x 48 x 16 blocks, 64 rays, map
 // and glossy query included); 4 take 303 us, being past 64 registers.
 template <class Args>
-__device__ __forceinline__ RayHit cast_ray_grid(const Args& a, f3 o, f3 d) {
+LUMX_HD RayHit cast_ray_grid(const Args& a, f3 o, f3 d) {
     const WorldView& w = a.world;
     const MarchRay m = march_ray(o, d);
     const int kx = w.wx + 2, kxy = kx * (w.wy + 2);
@@ -133,9 +142,9 @@ __device__ __forceinline__ RayHit cast_ray_grid(const Args& a, f3 o, f3 d) {
         int taken = 0;
         do {
             s0 = sample(fraction);
-            b0 = gld(a.grid, (unsigned)fminf(s0.index, last));
+            b0 = gld(a.grid, clamp_index(s0.index, last));
             s1 = sample(s0.next);
-            b1 = gld(a.grid, (unsigned)fminf(s1.index, last));
+            b1 = gld(a.grid, clamp_index(s1.index, last));
             second = b0 == 0 && s0.next < a.max_dist && left > taken + 1;
             on = second && b1 == 0 && s1.next < a.max_dist && left > taken + 2;
             fraction = s1.next;
@@ -162,7 +171,7 @@ __device__ __forceinline__ RayHit cast_ray_grid(const Args& a, f3 o, f3 d) {
             auto leaves = [&]() {
                 return fminf(pos.x, fminf(pos.y, pos.z)) < 0.0f || fraction >= a.max_dist || left == 0;
             };
-            key = bx + __mul24(by, kx) + __mul24(bz, kxy);
+            key = bx + (int)(mul24((unsigned)by, (unsigned)kx) + mul24((unsigned)bz, (unsigned)kxy));
             if (voxels && gld(w.palette, slot | voxel_offset(ix, iy, iz)) != 0) state = 1;
             else if (leaves()) state = -1;
             bool same = true;
