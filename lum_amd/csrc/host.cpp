@@ -321,8 +321,8 @@ void* lumx_context_stream(lumx_context_t c) { return c ? (void*)c->stream : null
 // the blocks to the last palette slot in use (its "static" state: serving
 // only changes fields, so a server copies that range out once).
 struct WorldLayout {
-    size_t blocks, copy_src, mats, palette, field0, field1, empty_bits, pal_bits, batch_counter, sel_bits,
-        sel_tiles, block_claim, upd_claim, upd_tiles, origin, blockify_state, total;
+    size_t blocks, copy_src, mats, palette, field0, field1, empty_bits, pal_bits, slot_mask, batch_counter,
+        sel_bits, sel_tiles, block_claim, upd_claim, upd_tiles, origin, blockify_state, total;
 };
 
 static WorldLayout world_layout(const lumx_world* w) {
@@ -343,6 +343,7 @@ static WorldLayout world_layout(const lumx_world* w) {
     L.field1 = take(nb * w->texel_bytes);
     L.empty_bits = take(((nb + 31) / 32) * sizeof(uint32_t));
     L.pal_bits = take(slots * 128 * sizeof(uint32_t));
+    L.slot_mask = take(slots);
     L.batch_counter = take(2 * sizeof(unsigned int));
     L.sel_bits = take(lumx::select_bits_bytes(w->n_blocks));
     L.sel_tiles = take(lumx::select_tiles(w->n_blocks) * sizeof(int));
@@ -376,12 +377,12 @@ static void world_carve(lumx_world* w, char* base) {
     const bool fits = nb + padded <= 4 * nb && padded <= (1 << 24);
     w->escape = fits ? (uint8_t*)w->block_claim : nullptr;
     w->grid = fits ? w->escape + nb : nullptr;
-    // Octants of the slots, where they fit as well (worlds in which the march's
-    // margin of 1/256 voxel covers the rounding of positions).
+    // Octants of the slots, for worlds in which the march's margin of 1/256 voxel
+    // covers the rounding of positions.  A place of their own: in the claim
+    // words every device map would have to read each static slot again (4 KiB a
+    // slot: 8 us for 16,384 slots).
     const int* ws = w->desc.size;
-    w->slot_mask = fits && nb + padded + w->desc.palette_slots <= 4 * nb && std::max(ws[0], std::max(ws[1], ws[2])) <= 512
-                       ? w->grid + padded
-                       : nullptr;
+    w->slot_mask = fits && std::max(ws[0], std::max(ws[1], ws[2])) <= 512 ? (uint8_t*)(base + L.slot_mask) : nullptr;
     w->upd_claim = (int*)(base + L.upd_claim);
     w->upd_tiles = (int*)(base + L.upd_tiles);
     w->origin_dev = (int16_t*)(base + L.origin);
@@ -1373,10 +1374,12 @@ static int map_device(lumx_world_t w, int n, const lumx_model_t* models, const l
     const int rc = [&]() -> int {
         HIP_TRY(launch_blockify(a, bound - st, s));
         if (int e = launch_models(w, n, models, pl, s)) return e;
-        // The claims took the place of every slot's mask.
-        const int from = w->slot_mask ? 0 : st, fill = w->slot_mask ? slots : 0;
+        // Slots above count as full: when this is a recorded map, the origin
+        // world of a later replay may name them.
         const int named = std::max(bound, w->origin_slots);
-        HIP_TRY(launch_palette_bits(w->palette, from, named - from, w->pal_bits, w->slot_mask, fill, s));
+        if (named > st)
+            HIP_TRY(launch_palette_bits(w->palette, st, named - st, w->pal_bits, w->slot_mask,
+                                        w->slot_mask ? slots : 0, s));
         GridArgs ga = grid_args(w);
         ga.slots = named;
         HIP_TRY(launch_march_grid(ga, s));

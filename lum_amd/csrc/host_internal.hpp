@@ -109,7 +109,8 @@ struct lumx_world {
     int* block_claim = nullptr;
     uint8_t* grid = nullptr;
     uint8_t* escape = nullptr;
-    uint8_t* slot_mask = nullptr;
+    uint8_t* slot_mask = nullptr;           // per slot: octants with a voxel (nullptr: worlds without a grid or an
+                                            // axis beyond 512 blocks)
     int* upd_claim = nullptr;               // per probe: last request of a subset update that
                                             // named it (-1 between updates)
     int* upd_tiles = nullptr;               // compacted subset update: per tile of 2048 probes
