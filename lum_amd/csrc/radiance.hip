@@ -651,44 +651,65 @@ hipError_t launch_radiance_refill(const RadianceArgs& a, int store, int P, hipSt
 
 // Many worlds in one launch.  World w owns threads [begin[w], begin[w+1]),
 // each range starting on a workgroup boundary; a workgroup finds its world by
-// a scalar binary search over begin[].  The per-probe arithmetic, RNG keying
-// (request index within the world's own update) and reduction order are those
-// of a single-world launch, so every world's result is the same alone and in
-// the batch.  time_seed of every world is offset by *frame (0 when null).
-// SERVED only separates the serving engine's launches from the batch API's
-// in profiles; the code is the same.
-template <int STORE, bool OCC, bool SERVED, int K>
+// last_begin().  The per-probe arithmetic, RNG keying (request index within
+// the world's own update) and reduction order are those of a single-world
+// launch, so every world's result is the same alone and in the batch.
+// time_seed of every world is offset by *frame (0 when null).  SERVED only
+// separates the serving engine's launches from the batch API's in profiles;
+// the code is the same.
+//
+// Arguments are constants (no thread writes them): each is loaded where it is
+// used and takes no register before.  A copy held 106 scalar registers, six
+// waves a SIMD: 2672 us for 24 worlds, 2389 us without it.
+struct BatchItem {
+    const RadianceArgs& a;
+    int time_seed;
+    uint32_t tid;  // within the world's range
+};
+__device__ __forceinline__ BatchItem batch_item(const RadianceArgs* args, const int* begin, int n_worlds,
+                                                const int* frame) {
+    const int b0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * blockDim.x));
+    const int lo = last_begin(begin, n_worlds, b0);
+    const RadianceArgs& a = *constant_args(args + lo);
+    return {a, a.time_seed + (frame ? *frame : 0), blockIdx.x * blockDim.x + threadIdx.x - (uint32_t)begin[lo]};
+}
+
+// One ray per lane, eight waves a SIMD like the single-world launch, although
+// the second body (fewer than 64 rays) then spills one to three registers:
+// 24 worlds of 48 x 48 x 16 blocks at 64 rays take 930 us, 979 us with 67
+// registers and seven waves.
+template <int STORE, bool SERVED>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(8)))
 radiance_batch_kernel(const RadianceArgs* args, const int* begin, int n_worlds, const int* frame) {
     extern __shared__ f3 chunk_sum[];
-    const int b0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * blockDim.x));
-    const int lo = last_begin(begin, n_worlds, b0);
-    // Arguments as constants (no thread writes them): each is loaded where it
-    // is used and takes no register before.  A copy held 106 scalar registers,
-    // six waves a SIMD: 2672 us for 24 worlds, 2389 us without it.
-    const RadianceArgs& a = *constant_args(args + lo);
-    const int time_seed = a.time_seed + (frame ? *frame : 0);
-    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x - (uint32_t)begin[lo];
-    if constexpr (K == 1 && !OCC) {
-        if (a.rays >= 64) radiance_chunk_body<STORE, true>(a, time_seed, tid, chunk_sum);
-        else radiance_chunk_body<STORE, false>(a, time_seed, tid, chunk_sum);
-    } else {
-        radiance_lane_body<STORE, false, OCC, K>(a, time_seed, tid, chunk_sum);
-    }
+    const BatchItem b = batch_item(args, begin, n_worlds, frame);
+    if (b.a.rays >= 64) radiance_chunk_body<STORE, true>(b.a, b.time_seed, b.tid, chunk_sum);
+    else radiance_chunk_body<STORE, false>(b.a, b.time_seed, b.tid, chunk_sum);
+}
+
+// Several rays per lane.  These need 71 to 85 registers: held to 64 they spill
+// 6 to 16, which large launches hide (1,141 us instead of 1,218 at two rays a
+// lane in the worlds above) and small ones do not (24 worlds of 16 x 16 x 8
+// blocks at 16 rays: 55 us instead of 46 at four rays a lane).
+template <int STORE, bool SERVED, int K>
+__global__ void __launch_bounds__(1024)
+radiance_batch_lanes_kernel(const RadianceArgs* args, const int* begin, int n_worlds, const int* frame) {
+    extern __shared__ f3 chunk_sum[];
+    const BatchItem b = batch_item(args, begin, n_worlds, frame);
+    radiance_lane_body<STORE, false, false, K>(b.a, b.time_seed, b.tid, chunk_sum);
 }
 
 template <int STORE, bool SERVED>
 static void launch_batch_k(int K, dim3 grid, dim3 block, size_t lds, hipStream_t stream, const RadianceArgs* args,
                            const int* begin, int n, const int* frame) {
     if (K == 4)
-        hipLaunchKernelGGL((radiance_batch_kernel<STORE, false, SERVED, 4>), grid, block, lds, stream, args, begin,
-                           n, frame);
+        hipLaunchKernelGGL((radiance_batch_lanes_kernel<STORE, SERVED, 4>), grid, block, lds, stream, args, begin, n,
+                           frame);
     else if (K == 2)
-        hipLaunchKernelGGL((radiance_batch_kernel<STORE, false, SERVED, 2>), grid, block, lds, stream, args, begin,
-                           n, frame);
+        hipLaunchKernelGGL((radiance_batch_lanes_kernel<STORE, SERVED, 2>), grid, block, lds, stream, args, begin, n,
+                           frame);
     else
-        hipLaunchKernelGGL((radiance_batch_kernel<STORE, false, SERVED, 1>), grid, block, lds, stream, args, begin,
-                           n, frame);
+        hipLaunchKernelGGL((radiance_batch_kernel<STORE, SERVED>), grid, block, lds, stream, args, begin, n, frame);
 }
 
 hipError_t launch_radiance_batch(const RadianceArgs* args_dev, const int* begin_dev, int n_worlds,
