@@ -33,18 +33,28 @@ FLAGS = [
 ]
 
 
-def build(verbose: bool = False) -> str:
-    srcs = [os.path.join(CSRC, s) for s in SOURCES]
-    tmp = OUT + ".tmp"
+def _compile(srcs, out: str, verbose: bool) -> str:
+    tmp = out + ".tmp"
     cmd = [HIPCC] + FLAGS + ["-x", "hip"] + srcs + ["-o", tmp]
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         sys.stderr.write(r.stdout + r.stderr)
-        raise RuntimeError("hipcc failed building liblumx.so")
-    os.replace(tmp, OUT)
-    return OUT
+        raise RuntimeError("hipcc failed building " + os.path.basename(out))
+    os.replace(tmp, out)
+    return out
+
+
+def build(verbose: bool = False) -> str:
+    return _compile([os.path.join(CSRC, s) for s in SOURCES], OUT, verbose)
+
+
+def build_tests(verbose: bool = False) -> str:
+    """tests/libmarch_device.so: the kernels' arithmetic over arrays, for the
+    GPU tests that compare it with IEEE arithmetic."""
+    tests = os.path.join(ROOT, "tests")
+    return _compile([os.path.join(tests, "march_device.hip")], os.path.join(tests, "libmarch_device.so"), verbose)
 
 
 if __name__ == "__main__":

@@ -68,8 +68,8 @@ LUMX_HD float dot3(f3 a, f3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 // rounded one, and a residual step takes a quotient within 1 ulp to the
 // correctly rounded one (the step before it brings a * inv there).  Checked
 // against IEEE division on gfx950 for every significand of d in rcp_rn, and
-// for 2^36 pairs in div_rn.  Three quotients by one divisor cost 18
-// instructions instead of 30.
+// for 2^36 pairs in div_rn (tests/test_gpu_arithmetic.py: 2^25).  Three
+// quotients by one divisor cost 18 instructions instead of 30.
 constexpr float kTiny = 0x1p-60f, kHuge = 0x1p60f;
 
 // 1 / d for kTiny <= |d| <= kHuge.
@@ -82,8 +82,9 @@ LUMX_HD float rcp_rn(float d) {
 #endif
 }
 
-// a / d for kTiny <= |d| <= kHuge and a = 0 or kTiny <= |a| <= kHuge, with
-// inv = 1 / d correctly rounded.
+// a / d for kTiny <= |d| <= kHuge and a = +0 or kTiny <= |a| <= kHuge, with
+// inv = 1 / d correctly rounded.  (-0 over a positive d gives +0; the callers'
+// numerators are differences and sums, which are never -0, or positive.)
 LUMX_HD float div_rn(float a, float d, float inv) {
 #if defined(__HIP_DEVICE_COMPILE__)
     float q = a * inv;
