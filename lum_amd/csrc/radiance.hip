@@ -61,8 +61,8 @@ __device__ __forceinline__ int dispatched_probes(const RadianceArgs& a) {
     return min(a.n_probes, gld(a.n_requests_dev, 0) / a.size);
 }
 
-// Probe wg's block coordinates (from the request list, the x-fastest index
-// or the compacted list) and the request index that keys its rays (wg, or
+// Probe wg's block coordinates (entry wg * size + shift of the request list or
+// of the x-fastest order, or the compacted list's) and the request index that keys its rays (wg, or
 // the entry's for a compacted update); false when outside the world or not
 // dispatched.
 __device__ __forceinline__ bool probe_coords(const RadianceArgs& a, int wg, int* px, int* py, int* pz, int* key) {
@@ -81,7 +81,7 @@ __device__ __forceinline__ bool probe_coords(const RadianceArgs& a, int wg, int*
         *py = q.y;
         *pz = q.z;
     } else {
-        probe_xyz(a, (uint32_t)wg, px, py, pz);
+        probe_xyz(a, (uint32_t)(wg * a.size + a.shift), px, py, pz);
     }
     const WorldView& w = a.world;
     return (unsigned)*px < (unsigned)w.wx && (unsigned)*py < (unsigned)w.wy && (unsigned)*pz < (unsigned)w.wz;
@@ -1207,7 +1207,7 @@ __global__ void __launch_bounds__(1024) radiance_tiled_kernel(RadianceArgs a) {
                     py = rq.y;
                     pz = rq.z;
                 } else {
-                    probe_xyz(a, (uint32_t)wg, &px, &py, &pz);
+                    probe_xyz(a, (uint32_t)(wg * a.size + a.shift), &px, &py, &pz);
                 }
                 valid = (unsigned)px < (unsigned)wv.wx && (unsigned)py < (unsigned)wv.wy &&
                         (unsigned)pz < (unsigned)wv.wz;
@@ -1271,7 +1271,7 @@ __global__ void __launch_bounds__(1024) radiance_tiled_kernel(RadianceArgs a) {
                 py = rq.y;
                 pz = rq.z;
             } else {
-                probe_xyz(a, (uint32_t)wg, &px, &py, &pz);
+                probe_xyz(a, (uint32_t)(wg * a.size + a.shift), &px, &py, &pz);
             }
             if ((unsigned)px >= (unsigned)wv.wx || (unsigned)py >= (unsigned)wv.wy || (unsigned)pz >= (unsigned)wv.wz)
                 continue;
