@@ -528,8 +528,11 @@ int lumx::world_snapshot_async(lumx_world* w, hipStream_t s, bool field_only) {
 }
 
 int lumx::world_snapshot_static(lumx_world* w) {
+    // The slots in use after a device map: an eviction compares them.
+    int rc = sync_host_state(w);
+    if (rc) return rc;
     const int used = kept_slots(w);
-    int rc = world_snapshot_reserve(w, used, nullptr);
+    rc = world_snapshot_reserve(w, used, nullptr);
     if (rc) return rc;
     HIP_TRY(hipMemcpy(w->snap_host, w->dev_mem, snap_static_bytes(w, used), hipMemcpyDeviceToHost));
     w->snap_used = used;
