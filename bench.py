@@ -519,7 +519,8 @@ def run_serving(args):
         w.restore()
     batch = Batch(ctx, worlds)
     batch.set_shape(served_block, served_rpl)
-    kernel_name = "radiance_batch_kernel<1,false,false,%d>" % served_rpl
+    kernel_name = ("radiance_batch_kernel<1,false>" if served_rpl == 1 else
+                   "radiance_batch_lanes_kernel<1,false,%d>" % served_rpl)
     rp = [radiance_params(rays=64, time_seed=0, alpha=0.1, max_steps=max_steps) for _ in worlds]
     bytes_per_launch = 0
     for w in worlds:

@@ -97,9 +97,11 @@ LUMX_HD unsigned clamp_index(float index, float last) {
 //   - The fraction: adding 1/2 is exact but where the result enters the next
 //     binade, and it does so once (n + 1 samples at most double it); rounding
 //     there commutes with adding multiples of 1/2.
-// Elsewhere the next kAhead samples are loaded together: 2 take 288 us where
-// 1 takes 320 us for a world with 32 models (48 x 48 x 16 blocks, 64 rays, map
-// and glossy query included); 4 take 303 us, being past 64 registers.
+// Elsewhere the next kAhead samples are loaded together.  A world with 32 models
+// (48 x 48 x 16 blocks, 64 rays, map and glossy query included) took 320 us
+// with 1, 288 with 2 and 303 with 4, which is past 64 registers (measured
+// before the air loop counted its samples per wave and before the selection
+// and blockify passes were cut; the same frame takes 236 us now, with 2).
 template <class Args>
 LUMX_HD RayHit cast_ray_grid(const Args& a, f3 o, f3 d) {
     const WorldView& w = a.world;

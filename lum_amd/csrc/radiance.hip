@@ -1389,7 +1389,7 @@ hipError_t launch_block_bits(const int16_t* blocks, int n_blocks, uint32_t* bits
     return hipGetLastError();
 }
 
-// March grid of a world (lumx_internal.hpp, MarchGrid) from its empty-block
+// March grid of a world (lumx_internal.hpp, GridArgs) from its empty-block
 // bits and its slots' octants.  A workgroup takes 32 x 4 x 4 blocks: the rows
 // of the tile and of the 8 blocks around it as 64-bit words of "not empty"
 // bits (bit 8 is the tile's first block), windowed along x with shifts, then
