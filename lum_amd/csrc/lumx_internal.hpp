@@ -83,12 +83,17 @@ struct GridArgs {
     int tiles;              // march_grid_tiles(wx, wy, wz)
 };
 #if defined(__HIPCC__)
+// The four octants with a voxel of a slot's half z < 8 or z >= 8, from its 64
+// occupancy words (one a lane).
+__device__ __forceinline__ unsigned half_octants(uint32_t word) {
+    const unsigned long long y0 = 0x0f0f0f0f0f0f0f0full;  // words of rows y < 8
+    const unsigned long long lo = __ballot((word & 0x00ff00ffu) != 0), hi = __ballot((word & 0xff00ff00u) != 0);
+    return ((lo & y0) != 0) | ((hi & y0) != 0) << 1 | ((lo & ~y0) != 0) << 2 | ((hi & ~y0) != 0) << 3;
+}
 // Octants of a slot with a voxel, from its occupancy words (128 threads).
 __device__ __forceinline__ void slot_octants(uint32_t word, int slot, uint8_t* slot_mask) {
     __shared__ unsigned upper;
-    const unsigned long long y0 = 0x0f0f0f0f0f0f0f0full;  // words of rows y < 8
-    const unsigned long long lo = __ballot((word & 0x00ff00ffu) != 0), hi = __ballot((word & 0xff00ff00u) != 0);
-    const unsigned m = ((lo & y0) != 0) | ((hi & y0) != 0) << 1 | ((lo & ~y0) != 0) << 2 | ((hi & ~y0) != 0) << 3;
+    const unsigned m = half_octants(word);
     if (threadIdx.x == 64) upper = m << 4;
     __syncthreads();
     if (threadIdx.x == 0) slot_mask[slot] = (uint8_t)(m | upper);

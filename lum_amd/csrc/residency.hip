@@ -13,16 +13,15 @@ namespace lumx {
 
 namespace {
 
-// One world's pass over the concatenation of five index ranges: elements
-// first, first + stride, ...; `lead` (one thread of the world's threads)
-// also resets the counters.
+// One world's pass over its slots, then over the concatenation of four index
+// ranges: elements first, first + stride, ...; `lead` (one thread of the
+// world's threads) also resets the counters.
 __device__ __forceinline__ void attach_world(const AttachArgs& a, long long first, long long stride, bool lead) {
     const long long n_field = a.n_field_words;
     const long long n_pal = (long long)(a.slots - a.used) * 512;  // uint2 words of the unused slots
     const long long n_claim = a.n_blocks;
     const long long n_eb = (a.n_blocks + 31) / 32;
-    const long long n_pb = (long long)a.slots * 128;
-    const long long total = n_field + n_pal + n_claim + n_eb + n_pb;
+    const long long total = n_field + n_pal + n_claim + n_eb;
     if (lead) {
         a.batch_counter[0] = 0;
         a.batch_counter[1] = 0;
@@ -31,27 +30,32 @@ __device__ __forceinline__ void attach_world(const AttachArgs& a, long long firs
         a.blockify_state[2] = 0;
         a.blockify_state[3] = 0;
     }
-    // Eight lanes a slot, one octant each (first is a thread's number and the
-    // stride a multiple of 64, so the lanes of a slot sit side by side).
-    const long long n_oct = a.slot_mask ? (long long)a.slots * 8 : 0;
-    for (long long i = first; i < n_oct; i += stride) {
-        const int slot = (int)(i >> 3), oct = (int)(i & 7);
-        bool any = false;
+    // Occupancy words and octants of the slots, a wave a slot (first is a
+    // thread's number and the stride a multiple of 64): a lane takes a word of
+    // the half z < 8 and one of the half above.  (Octants by lanes of their own,
+    // each reading a slot's eighth, were a chain of loads beside the other work:
+    // a 64 x 64 x 16 world 9.2 us, 7.2 without octants.)
+    const int lane = (int)(threadIdx.x & 63);
+    for (long long i = first; i < (long long)a.slots * 64; i += stride) {
+        const int slot = (int)(i >> 6);
+        uint32_t v[2] = {0u, 0u};
         if (slot < a.used) {
-            const uint8_t* src = a.palette + ((size_t)slot << 12) + ((oct & 1) << 3) + ((oct & 2) << 6) + ((oct & 4) << 9);
-            uint2 v = make_uint2(0u, 0u);
-            for (int z = 0; z < 8; ++z) {
+            const uint4* src = (const uint4*)(a.palette + ((size_t)slot << 12) + lane * 32);
 #pragma unroll
-                for (int y = 0; y < 8; ++y) {
-                    const uint2 r = *(const uint2*)(src + z * 256 + y * 16);
-                    v.x |= r.x;
-                    v.y |= r.y;
-                }
+            for (int h = 0; h < 2; ++h) {
+                const uint4 a0 = src[h * 128], a1 = src[h * 128 + 1];
+                const uint32_t w[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+#pragma unroll
+                for (int k = 0; k < 32; ++k) v[h] |= (((w[k >> 2] >> ((k & 3) * 8)) & 0xffu) != 0 ? 1u : 0u) << k;
             }
-            any = (v.x | v.y) != 0;
         }
-        const unsigned long long b = __ballot(any);
-        if (oct == 0) a.slot_mask[slot] = (uint8_t)(b >> (threadIdx.x & 56));
+        uint32_t* bits = a.pal_bits + ((size_t)slot << 7) + lane;
+        bits[0] = v[0];
+        bits[64] = v[1];
+        if (a.slot_mask) {
+            const unsigned m = half_octants(v[0]) | half_octants(v[1]) << 4;
+            if (lane == 0) a.slot_mask[slot] = (uint8_t)m;
+        }
     }
     for (long long i = first; i < total; i += stride) {
         long long j = i;
@@ -70,25 +74,10 @@ __device__ __forceinline__ void attach_world(const AttachArgs& a, long long firs
             continue;
         }
         j -= n_claim;
-        if (j < n_eb) {
-            const long long base = j * 32;
-            uint32_t v = 0;
-            for (int k = 0; k < 32 && base + k < a.n_blocks; ++k) v |= (a.blocks[base + k] == 0 ? 1u : 0u) << k;
-            a.empty_bits[j] = v;
-            continue;
-        }
-        j -= n_eb;
-        // pal_bits word j: slot j / 128, voxels 32 (j % 128) .. + 31
-        const int slot = (int)(j >> 7);
+        const long long base = j * 32;
         uint32_t v = 0;
-        if (slot < a.used) {
-            const uint4* src = (const uint4*)(a.palette + ((size_t)j << 5));
-            const uint4 a0 = src[0], a1 = src[1];
-            const uint32_t w[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-#pragma unroll
-            for (int k = 0; k < 32; ++k) v |= (((w[k >> 2] >> ((k & 3) * 8)) & 0xffu) != 0 ? 1u : 0u) << k;
-        }
-        a.pal_bits[j] = v;
+        for (int k = 0; k < 32 && base + k < a.n_blocks; ++k) v |= (a.blocks[base + k] == 0 ? 1u : 0u) << k;
+        a.empty_bits[j] = v;
     }
 }
 
